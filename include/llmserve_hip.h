@@ -131,6 +131,24 @@ int llmserve_int4_linear_gemm(const float* x, const float* inv_act_scale /* null
                               void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * Int4 linear for batches past the decode sizes, any group_size multiple of 64 (Int4Linear's
+ * large-M branch, quant.py:141-142): x' = x * inv_act_scale is split into two fp16 pieces of a
+ * row scaled by a power of two (22 significant bits down to 2^-38 of the row's largest value),
+ * every matrix-core product is exact and summed in fp32. `packed` is nullable: the buffer of
+ * llmserve_int4_gemm_pack for the same weight (group_size a multiple of 128), which spares the
+ * call its own repacking of the nibbles. Requires K % 128 == 0, 16-byte aligned x,
+ * inv_act_scale, nibbles and packed, and a 16-byte aligned workspace of
+ * llmserve_int4_linear_tile_workspace_bytes(M, N, K, group_size) bytes.
+ */
+int64_t llmserve_int4_linear_tile_workspace_bytes(int64_t M, int64_t N, int64_t K,
+                                                  int64_t group_size);
+int llmserve_int4_linear_tile(const float* x, const float* inv_act_scale /* nullable [K] */,
+                              const uint8_t* nibbles, const float* g_scale, const float* g_zero,
+                              const void* packed /* nullable */, float* y, int64_t M, int64_t N,
+                              int64_t K, int64_t group_size, void* workspace,
+                              int64_t workspace_bytes, void* stream);
+
+/*
  * The weights of llmserve_int4_linear_gemm_packed: nibbles, group scales and zeros of
  * llmserve_int4_quantize rearranged once (per weight, at load time) into the order the
  * matrix-core kernel reads them, so that each of its load instructions reads contiguous bytes

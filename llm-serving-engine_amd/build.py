@@ -54,6 +54,7 @@ HIP_SOURCES = [
     "gemv.hip",
     "gemm_prefill.hip",
     "gemm_int4.hip",
+    "gemm_tile.hip",
     "fused_ops.hip",
     "sampling.hip",
     "paged_decode.hip",

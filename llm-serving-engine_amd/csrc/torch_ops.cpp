@@ -212,6 +212,65 @@ at::Tensor int4_linear_gemm(const at::Tensor& x, const at::Tensor& nibbles, cons
   return y;
 }
 
+void check_int4_tile(const at::Tensor& x, const at::Tensor& nibbles, const at::Tensor& scale,
+                     const at::Tensor& zero, int64_t group_size,
+                     const std::optional<at::Tensor>& inv_act_scale) {
+  TORCH_CHECK(x.scalar_type() == at::kFloat && nibbles.scalar_type() == at::kByte &&
+                  scale.scalar_type() == at::kFloat && zero.scalar_type() == at::kFloat,
+              "int4_linear_tile: dtypes");
+  TORCH_CHECK(x.dim() == 2 && nibbles.dim() == 2 && group_size > 0 &&
+                  nibbles.size(1) * 2 == x.size(1) && x.size(1) % group_size == 0 &&
+                  scale.numel() == nibbles.size(0) * (x.size(1) / group_size) &&
+                  zero.numel() == scale.numel(),
+              "int4_linear_tile: shapes");
+  if (inv_act_scale.has_value())
+    TORCH_CHECK(inv_act_scale->scalar_type() == at::kFloat && inv_act_scale->numel() == x.size(1),
+                "int4_linear_tile: inv_act_scale must be a float32 [K] tensor");
+}
+
+at::Tensor int4_linear_tile(const at::Tensor& x, const at::Tensor& nibbles, const at::Tensor& scale,
+                            const at::Tensor& zero, int64_t group_size,
+                            const std::optional<at::Tensor>& inv_act_scale,
+                            const std::optional<at::Tensor>& packed) {
+  check_int4_tile(x, nibbles, scale, zero, group_size, inv_act_scale);
+  TORCH_CHECK(x.is_contiguous() && nibbles.is_contiguous() && scale.is_contiguous() &&
+                  zero.is_contiguous() && (!inv_act_scale.has_value() || inv_act_scale->is_contiguous()),
+              "int4_linear_tile: contiguous inputs");
+  check_device(x, {&nibbles, &scale, &zero}, "int4_linear_tile");
+  if (inv_act_scale.has_value()) check_device(x, {&*inv_act_scale}, "int4_linear_tile");
+  const int64_t M = x.size(0), K = x.size(1), N = nibbles.size(0);
+  if (packed.has_value()) {
+    check_device(x, {&*packed}, "int4_linear_tile");
+    TORCH_CHECK(packed->scalar_type() == at::kByte && packed->is_contiguous() &&
+                    packed->numel() == llmserve_int4_gemm_pack_bytes(N, K, group_size),
+                "int4_linear_tile: packed is not int4_gemm_pack's buffer for this weight");
+  }
+  const c10::DeviceGuard guard(x.device());
+  // a view at an odd offset is copied: the kernel reads 16-byte pieces
+  auto aligned = [](const at::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.clone();
+  };
+  const at::Tensor xa = aligned(x), na = aligned(nibbles);
+  std::optional<at::Tensor> inv;
+  if (inv_act_scale.has_value()) inv = aligned(*inv_act_scale);
+  auto y = at::empty({M, N}, x.options());
+  const int64_t ws_bytes = llmserve_int4_linear_tile_workspace_bytes(M, N, K, group_size);
+  at::Tensor ws;
+  if (ws_bytes > 0) ws = at::empty({ws_bytes}, nibbles.options());
+  check_status(llmserve_int4_linear_tile(
+      xa.data_ptr<float>(), opt_ptr<float>(inv), na.data_ptr<uint8_t>(),
+      scale.data_ptr<float>(), zero.data_ptr<float>(), opt_ptr<uint8_t>(packed), y.data_ptr<float>(), M, N,
+      K, group_size, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(x)));
+  return y;
+}
+
+at::Tensor int4_linear_tile_meta(const at::Tensor& x, const at::Tensor& nibbles, const at::Tensor& scale,
+                                 const at::Tensor& zero, int64_t group_size,
+                                 const std::optional<at::Tensor>& inv_act_scale,
+                                 const std::optional<at::Tensor>& packed) {
+  return at::empty_symint({x.sym_size(0), nibbles.sym_size(0)}, x.options());
+}
+
 at::Tensor int4_gemm_pack(const at::Tensor& nibbles, const at::Tensor& scale,
                           const at::Tensor& zero, int64_t group_size) {
   TORCH_CHECK(nibbles.scalar_type() == at::kByte && scale.scalar_type() == at::kFloat &&
@@ -816,6 +875,8 @@ TORCH_LIBRARY(llmserve_hip, m) {
         " Tensor? inv_act_scale=None) -> Tensor");
   m.def("int4_linear_gemm(Tensor x, Tensor nibbles, Tensor scale, Tensor zero, int group_size,"
         " Tensor? inv_act_scale=None) -> Tensor");
+  m.def("int4_linear_tile(Tensor x, Tensor nibbles, Tensor scale, Tensor zero, int group_size,"
+        " Tensor? inv_act_scale=None, Tensor? packed=None) -> Tensor");
   m.def("int4_gemm_pack(Tensor nibbles, Tensor scale, Tensor zero, int group_size) -> Tensor");
   m.def("int4_linear_gemm_packed(Tensor x, Tensor packed, int out_features, int group_size,"
         " Tensor? inv_act_scale=None) -> Tensor");
@@ -864,6 +925,7 @@ TORCH_LIBRARY_IMPL(llmserve_hip, CUDA, m) {
   m.impl("int8_linear", &int8_linear);
   m.impl("int8_linear_prefill", &int8_linear_prefill);
   m.impl("int4_linear_gemm", &int4_linear_gemm);
+  m.impl("int4_linear_tile", &int4_linear_tile);
   m.impl("int4_gemm_pack", &int4_gemm_pack);
   m.impl("int4_linear_gemm_packed", &int4_linear_gemm_packed);
   m.impl("int4_linear", &int4_linear);
@@ -887,3 +949,6 @@ TORCH_LIBRARY_IMPL(llmserve_hip, CUDA, m) {
   m.impl("paged_attention_rows", &paged_attention_rows);
   m.impl("attention_metadata", &attention_metadata);
 }
+
+// Shapes for tracing (torch.compile, FakeTensor).
+TORCH_LIBRARY_IMPL(llmserve_hip, Meta, m) { m.impl("int4_linear_tile", &int4_linear_tile_meta); }

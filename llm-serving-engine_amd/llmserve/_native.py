@@ -55,6 +55,8 @@ C_SIGNATURES: dict[str, tuple[object, list]] = {
     "llmserve_int4_linear_gemm": (_I32, [_P] * 6 + [_I64] * 4 + [_P, _I64, _P]),
     "llmserve_int4_gemm_pack_bytes": (_I64, [_I64, _I64, _I64]),
     "llmserve_int4_gemm_pack": (_I32, [_P, _P, _P, _I64, _I64, _I64, _P, _I64, _P]),
+    "llmserve_int4_linear_tile_workspace_bytes": (_I64, [_I64] * 4),
+    "llmserve_int4_linear_tile": (_I32, [_P] * 7 + [_I64] * 4 + [_P, _I64, _P]),
     "llmserve_int4_linear_gemm_packed_workspace_bytes": (_I64, [_I64, _I64]),
     "llmserve_int4_linear_gemm_packed": (_I32, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _I64, _P]),
     "llmserve_int4_xfrag_bytes": (_I64, [_I64, _I64]),

@@ -14,8 +14,9 @@ Functions, with the reference's names and signatures where the reference has the
   zero, group_size, inv_act_scale=None)`` (int8_gemv.cpp:109-112; ``inv_act_scale`` fuses
   Int4Linear's AWQ pre-scale); ``int8_linear_prefill(x, qweight, scale)``, Int8Linear's
   large-M path on the bf16 matrix cores (quant.py:71-72); ``int4_linear_gemm(...)``,
-  Int4Linear's large-M path (quant.py:141-142); ``int4_gemm_pack(nibbles, scale, zero,
-  group_size)`` and ``int4_linear_gemm_packed(x, packed, out_features, group_size,
+  Int4Linear's large-M path on the reference layout (quant.py:141-142) and
+  ``int4_linear_tile(..., packed=None)``, the one it takes; ``int4_gemm_pack(nibbles, scale,
+  zero, group_size)`` and ``int4_linear_gemm_packed(x, packed, out_features, group_size,
   inv_act_scale=None)``, the decode-batch matrix-core kernel on a rearranged weight.
 * ``load_paged_attention()``: ``paged_attention_decode_int8(q, k_cache, v_cache, k_scale,
   v_scale, block_tables, context_lens, block_size, scale, partition_size=0, q_mult=None)`` and
@@ -99,7 +100,7 @@ def load_int8_gemv() -> SimpleNamespace | None:
     """Weight-only int8 / int4 matmuls (HIP, gfx950), or None."""
     return _namespace("int8/int4 GEMV kernels", (
         "int8_linear", "int4_linear", "int8_linear_prefill", "int4_linear_gemm",
-        "int4_gemm_pack", "int4_linear_gemm_packed"))
+        "int4_gemm_pack", "int4_linear_gemm_packed", "int4_linear_tile"))
 
 
 @functools.cache

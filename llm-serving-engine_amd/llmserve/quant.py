@@ -190,8 +190,9 @@ class Int4Linear(nn.Module):
     max_packed_rows = 256  # up to this: the decode-batch kernel on the packed weight
     # "auto": the HIP GEMV up to gemv_max_rows rows, the matrix-core kernel on the packed weight
     # ("gemm", K and group multiples of 128) up to max_packed_rows, the GEMV up to
-    # max_fused_rows when there is no packed weight, then the matrix-core GEMM on the reference
-    # layout ("gemm_ref") or dequantize + GEMM ("aten", the reference's large-M algorithm).
+    # max_fused_rows when there is no packed weight, then the tiled matrix-core GEMM (K a
+    # multiple of 128 and the group of 64; no explicit name) or dequantize + GEMM ("aten", the
+    # reference's large-M algorithm). "gemm_ref": the matrix-core GEMM on the reference layout.
     kernel = "auto"
 
     def __init__(
@@ -249,7 +250,16 @@ class Int4Linear(nn.Module):
         return (self.in_features % 128 == 0 and self.group_size % 128 == 0
                 and self.out_features % 16 == 0)
 
-    def _path(self, rows: int, native) -> str:
+    def _tile_ok(self, x: torch.Tensor) -> bool:
+        """Inputs the tiled GEMM (int4_linear_tile) takes; the others keep the torch ops, which
+        differentiate and promote types."""
+        rows, (n, k) = x.shape[0], (self.out_features, self.in_features)
+        return (k % 128 == 0 and self.group_size % 64 == 0 and x.dtype == torch.float32
+                and rows < 2**24 and n < 2**22 and k < 2**20 and rows * k < 2**36
+                and not (x.requires_grad and torch.is_grad_enabled())
+                and torch.autograd.forward_ad._current_level < 0)
+
+    def _path(self, rows: int, native, x: torch.Tensor | None = None) -> str:
         if self.kernel not in ("auto", "gemv", "gemm", "gemm_ref", "aten"):
             raise ValueError(f"unknown Int4Linear kernel {self.kernel!r}")
         if native is None:
@@ -263,6 +273,8 @@ class Int4Linear(nn.Module):
             return "gemm"
         if rows <= self.max_fused_rows:
             return "gemv"
+        if x is not None and self._tile_ok(x):
+            return "tile"
         if self.gemm_packed is not None and not self.gemm_ok():
             return "gemm"
         return "gemm_ref" if self.gemm_ok() else "aten"
@@ -271,7 +283,7 @@ class Int4Linear(nn.Module):
         lead = x.shape[:-1]
         x2 = x.reshape(-1, x.shape[-1])
         native = _native("gemv", x2.device)
-        path = self._path(x2.shape[0], native)
+        path = self._path(x2.shape[0], native, x2)
         if path == "aten":
             xs = x2 * self.inv_act_scale if self.inv_act_scale is not None else x2
             y = xs @ self.dequantize().t()
@@ -279,6 +291,9 @@ class Int4Linear(nn.Module):
             y = native.int4_linear_gemm_packed(x2.contiguous(), self.gemm_packed,
                                                self.out_features, self.group_size,
                                                self.inv_act_scale)
+        elif path == "tile":
+            y = native.int4_linear_tile(x2.contiguous(), self.nibbles, self.g_scale, self.g_zero,
+                                        self.group_size, self.inv_act_scale, self.gemm_packed)
         else:
             fn = native.int4_linear if path == "gemv" else native.int4_linear_gemm
             y = fn(x2.contiguous(), self.nibbles, self.g_scale, self.g_zero, self.group_size,

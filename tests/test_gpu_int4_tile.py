@@ -1,0 +1,99 @@
+"""The tiled int4 GEMM (llmserve_int4_linear_tile, Int4Linear's large-M path) against float64.
+
+Bound: x' is held to 2^-22 of each element (two fp16 pieces), the zero term's operands to 2^-22
+as well, and fp32 adds at most K / 32 partial sums of exact products: with random signs about
+2^-22 + 2^-24 sqrt(K / 32), below 1e-6 relative (2-norm) for K up to 8192; 2e-6 is asked, and ten
+times that of the largest value.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from llmserve.kernels import load_int8_gemv
+from oracle import math_ref as mr
+from oracle import quant as oq
+
+pytestmark = pytest.mark.gpu
+F32 = np.float32
+
+
+def make(seed, M, N, K, group, awq):
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((M, K)).astype(F32)
+    x[:, rng.permutation(K)[: max(1, K // 100)]] *= 20
+    act = (np.abs(rng.standard_normal(K)) + 0.2).astype(F32) if awq else None
+    w = (rng.standard_normal((N, K)) * 0.02).astype(F32)
+    return (x, *oq.int4_quantize_pack(w, group, act))
+
+
+def run(x, nib, gs, gz, group, inv, packed):
+    ops = load_int8_gemv()
+    t = [torch.from_numpy(a).cuda() if a is not None else None for a in (x, nib, gs, gz, inv)]
+    pk = ops.int4_gemm_pack(t[1], t[2], t[3], group) if packed else None
+    return ops.int4_linear_tile(t[0], t[1], t[2], t[3], group, t[4], pk), t
+
+
+def check(y, x, nib, gs, gz, group, inv):
+    ref = mr.int4_linear_f64(x, nib, gs, gz, group, inv)
+    y = y.cpu().numpy().astype(np.float64)
+    assert np.linalg.norm(y - ref) <= 2e-6 * np.linalg.norm(ref)
+    assert np.abs(y - ref).max() <= 2e-5 * np.abs(ref).max()
+
+
+# tile edges (16, 32, 64 rows; 64, 128, 256 channels), odd sizes, an odd count of K blocks, groups of
+# 64 / 128 / 192 / 256 / the whole row, more than 64 units of K, each tile of the dispatch
+@pytest.mark.parametrize("M,N,K,group,packed", [
+    (1, 1, 128, 64, False), (17, 63, 128, 128, False), (16, 64, 256, 64, False),
+    (33, 65, 384, 192, False), (31, 129, 640, 128, True), (65, 300, 1152, 64, False),
+    (129, 257, 512, 256, True), (100, 1000, 8320, 64, False), (70, 200, 1024, 1024, True),
+    (300, 1464, 1664, 128, True), (257, 4100, 256, 64, False), (513, 2049, 384, 128, False),
+    (1030, 6100, 256, 64, False), (1281, 4160, 384, 128, True)])
+def test_tile_vs_f64(gpu, M, N, K, group, packed):
+    x, nib, gs, gz, inv = make(M + N + K, M, N, K, group, M % 2 == 1)
+    y, t = run(x, nib, gs, gz, group, inv, packed)
+    check(y, x, nib, gs, gz, group, inv)
+    if packed:  # the caller's packing and the call's own give the same bits
+        assert torch.equal(y, run(x, nib, gs, gz, group, inv, False)[0])
+    off = torch.zeros(t[0].numel() + 1, device="cuda")[1:].view(t[0].shape)  # 4-byte aligned rows
+    off.copy_(t[0])
+    assert torch.equal(y, load_int8_gemv().int4_linear_tile(off, t[1], t[2], t[3], group, t[4]))
+
+
+def test_rows_are_independent_and_wide_ranges_hold(gpu):
+    """Rows of 1e-30 .. 1e30, a zero row, a row with a NaN and one with an infinity: each row's
+    result is its own, and finite rows keep their precision."""
+    x, nib, gs, gz, inv = make(5, 40, 96, 256, 64, True)
+    x[:8] *= np.logspace(-30, 30, 8).astype(F32)[:, None]
+    x[8] = 0
+    x[9, 3], x[10, 200] = np.nan, np.inf
+    y = run(x, nib, gs, gz, 64, inv, False)[0].cpu().numpy()
+    fine = [r for r in range(40) if r not in (9, 10)]
+    assert not np.isfinite(y[[9, 10]]).any() and not y[8].any()
+    ref = mr.int4_linear_f64(x[fine], nib, gs, gz, 64, inv)
+    err = np.linalg.norm(y[fine] - ref, axis=1)
+    assert (err <= 3e-6 * np.linalg.norm(ref, axis=1)).all()
+
+
+@pytest.mark.parametrize("group,rows,path", [(64, 16, "gemv"), (64, 17, "tile"), (128, 256, "gemm"),
+                                             (128, 257, "tile")])
+def test_module_dispatch(gpu, group, rows, path):
+    from llmserve.quant import Int4Linear
+
+    base = torch.nn.Linear(256, 200, device="cuda")
+    m = Int4Linear(base, group)
+    x = torch.randn(rows, 256, device="cuda")
+    assert m._path(rows, load_int8_gemv(), x) == path
+    with torch.inference_mode():
+        y = m(x)
+    ref = x.double() @ m.dequantize().double().t() + m.bias.double()
+    assert (y - ref).norm() <= 1e-5 * ref.norm()
+    # gradients, other types and K off the 128 grid keep the torch ops
+    xg = x.clone().requires_grad_()
+    assert m._path(rows, load_int8_gemv(), xg) != "tile"
+    assert not m._tile_ok(x.bfloat16())
+    assert not Int4Linear(torch.nn.Linear(192, 8, device="cuda"), 64)._tile_ok(x[:, :192])
+    assert torch.ops.llmserve_hip.int4_linear_tile(
+        *(t.to("meta") for t in (x, m.nibbles, m.g_scale, m.g_zero)), group).shape == y.shape
