@@ -421,6 +421,28 @@ int llmserve_paged_attention_decode(const float* q, const float* k_cache, const 
                                     int64_t workspace_bytes, void* stream);
 
 /*
+ * Causal attention of prompt tokens on the matrix cores (the prefill branch of the reference's
+ * paged_attention, attention.py:249-257): q / out [T, Hq, D], tiles [n_tiles, 4] int64 rows (first
+ * query row, query rows <= 64, context tokens the first row sees, block-table row); row i of a
+ * tile sees i more tokens than its first. `tiles` is in device memory, `tiles_host` the same
+ * values on the host (checked against the batch, and the launch is planned from them). int8
+ * caches with scales, or float32 caches with k_scale = v_scale = NULL. D = 64 or 128; q, caches and
+ * out 16-byte aligned. Query rows outside the tiles are left alone.
+ */
+int64_t llmserve_paged_attention_prefill_workspace_bytes(const int64_t* tiles_host,
+                                                         int64_t n_tiles, int64_t Hq, int64_t Hk,
+                                                         int64_t D);
+int llmserve_paged_attention_prefill(const float* q, const void* k_cache, const void* v_cache,
+                                     const float* k_scale, const float* v_scale,
+                                     const int64_t* block_tables, int64_t table_rows,
+                                     const int64_t* tiles, const int64_t* tiles_host,
+                                     int64_t n_tiles, float* out, int64_t T, int64_t Hq, int64_t Hk,
+                                     int64_t D, int64_t num_slots, int64_t max_blocks,
+                                     int64_t block_size, float scale,
+                                     const float* q_mult /* nullable [Hq, D] */, void* workspace,
+                                     int64_t workspace_bytes, void* stream);
+
+/*
  * Paged attention for the query rows of a ragged batch, decode and prefill alike (replaces
  * paged_attention's prefill loop and decode branch, attention.py:249-307, over the cache of
  * attention.py:241-246): query row r attends, with the paged decode's split and merge, to the

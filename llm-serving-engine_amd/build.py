@@ -58,6 +58,7 @@ HIP_SOURCES = [
     "fused_ops.hip",
     "sampling.hip",
     "paged_decode.hip",
+    "prefill_attn.hip",
     "attn_meta.hip",
     "decode_chain.hip",
     "lm_head.hip",

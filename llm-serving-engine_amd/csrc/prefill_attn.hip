@@ -1,0 +1,753 @@
+// Causal paged attention of prompt tokens on the fp16 matrix cores (the prefill branch of the
+// reference's paged_attention, attention.py:249-257, whose gather + SDPA this replaces), over the
+// int8 or the fp32 cache.
+//
+// The row kernel (paged_decode.hip) gives every token a query row of its own: it reads the whole
+// context once per token and runs on the VALU (2 prompts of ~900 tokens after ~1000 cached ones and 24
+// decode rows: 962 us). Here a workgroup takes 64 query tokens and two query heads of one kv head and
+// walks the context in tiles of 64 tokens (fp32 cache: 32) that its four wavefronts share: 87 us for
+// the two prompts, 1000 new tokens over the fp32 cache 776 -> 66.
+//
+// Precision is fp32's: q, the weights and fp32 K / V rows are each split into two fp16 pieces (22
+// bits) after scaling by a power of two (per query row and head, per cache row); int8 codes are exact
+// in fp16, their scales stay in fp32 on the score and on the weight. Products are exact and summed in
+// fp32. Measured against float64: 1.4-3.1e-7 (int8), the row kernel 3.0e-7.
+//
+// Both products are transposed: S^T = K Q^T leaves lane (fr, fc) the scores of query fr for tokens
+// 16 tt + 4 fc + e, which is the B operand layout of O^T = V^T P^T when the k order of that product is
+// chosen as those tokens. So the weights go from accumulator to operand in place, a query's running
+// reference and sum are per-lane scalars, and only a moving reference needs other lanes. V is
+// transposed on its way into LDS (4 tokens x 4 dims per thread with byte permutes).
+//
+// Each wavefront brings its own quarter of the next context tile straight into LDS while the
+// current one is computed, then widens it into MFMA fragments (positions in a fragment are permuted so
+// that neither the writes nor the reads conflict). Long contexts are split into chunks where the
+// tiles alone would leave CUs idle, and a second launch adds the chunks.
+// What bounds it: per context tile a wavefront issues 128 products (2048 matrix-core cycles) and ~410
+// VALU instructions (exp, the splits, widening); the two wavefronts of a SIMD overlap them only in
+// part: 8192 tokens run at 460 TFLOP/s of attention, 0.92 PFLOP/s of fp16 products.
+#include <algorithm>
+#include <type_traits>
+
+#include "common.h"
+
+namespace {
+
+using lsh::kWave;
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kQT = 64;         // query tokens of a tile: 16 per wavefront
+constexpr int kHeads = 2;       // query heads of a workgroup (of one kv head)
+constexpr int kWaves = 4;
+constexpr int kFrag = 1024;     // bytes of a fragment: 64 lanes x 8 fp16
+constexpr float kLog2e = 1.4426950408889634f;
+// Weights: p = exp2(score - ref), ref the running max of score + log2(v scale) (so that p v_scale
+// stays below 2^kLazy: the reference moves only past that), times v_scale kUp, which brings the fp16
+// pieces near the top of their range. kUp is a factor of the staged v scales rather than of p: p's
+// exponent stays small, and with it the rounding of its argument.
+constexpr float kLazy = 4.f, kUp = 2048.f;
+// A v scale that is not finite is staged as kHuge, so that a weight of 0 (a token that the query does
+// not see) times it stays 0; a weight that is not 0 still overflows fp16, as the reference follows
+// v scales up to 2^kMaxLv only, and the output is NaN.
+constexpr float kHuge = 3.402823466e38f, kMaxLv = 100.f;
+
+struct PrefillArgs {
+  const float* q;
+  const void* kc;
+  const void* vc;
+  const float* ks;
+  const float* vs;
+  const int64_t* bt;
+  const int64_t* tiles;  // [n][4]: first query row, query rows, tokens the first row sees, table row
+  const float* q_mult;
+  float* out;
+  float* part_acc;  // [tile][kv head, head pair][chunk][kHeads][kQT][D]
+  float* part_rl;   // [tile][kv head, head pair][chunk][kHeads][kQT][2] (reference, sum)
+  int64_t num_slots;
+  int n_tiles, Hq, Hk, G, pairs;  // pairs: head pairs of a kv head
+  int max_blocks, bs, bs_shift;
+  int chunk, splits;  // most tokens of a context chunk (a multiple of 64), most chunks of a tile
+  float scale;
+};
+
+__device__ __forceinline__ f16x2 as_h2(uint32_t w) { return __builtin_bit_cast(f16x2, w); }
+__device__ __forceinline__ uint32_t as_u(f16x2 h) { return __builtin_bit_cast(uint32_t, h); }
+__device__ __forceinline__ f32x4 mfma(const f16x8& a, const f16x8& b, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// Max over the lanes with the same lane % 16.
+__device__ __forceinline__ float max_over_fc(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  v = fmaxf(__builtin_bit_cast(float, static_cast<uint32_t>(a[0])), __builtin_bit_cast(float, static_cast<uint32_t>(a[1])));
+  const uint32_t w = __builtin_bit_cast(uint32_t, v);
+  const auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+  return fmaxf(__builtin_bit_cast(float, static_cast<uint32_t>(b[0])), __builtin_bit_cast(float, static_cast<uint32_t>(b[1])));
+}
+__device__ __forceinline__ float sum_over_fc(float v) {
+  v += __shfl_xor(v, 16, kWave);
+  return v + __shfl_xor(v, 32, kWave);
+}
+
+__device__ __forceinline__ int exponent_to_15(float top) {  // 2^result brings top to [2^14, 2^15)
+  int ex = 0;
+  if (top > 0.f && top < __builtin_inff()) ex = 15 - __builtin_amdgcn_frexp_expf(top);
+  return ex < -126 ? -126 : (ex > 126 ? 126 : ex);
+}
+
+// Two values -> packed hi and lo pieces. The empty asm makes hi one value: left to itself the
+// compiler converts a second time for lo's subtraction (fused with the product that made the
+// value, which rounds differently).
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  hi = as_u(__builtin_convertvector(f32x2{a, b}, f16x2));
+  asm("" : "+v"(hi));
+  const f16x2 h = as_h2(hi);
+  const f16x2 l = {static_cast<_Float16>(__builtin_fmaf(a, 1.f, -static_cast<float>(h[0]))),
+                   static_cast<_Float16>(__builtin_fmaf(b, 1.f, -static_cast<float>(h[1])))};
+  lo = as_u(l);
+}
+
+// bytes b0, b1 of `pair` (each value + 128) -> two fp16 values, exact
+template <uint32_t SEL>
+__device__ __forceinline__ uint32_t bytes_to_h2(uint32_t w) {
+  const f16x2 k = {1152, 1152};
+  return as_u(as_h2(__builtin_amdgcn_perm(0x64646464u, w, SEL)) - k);
+}
+
+// Tokens of the chunks of a context: as few chunks of at most `most` tokens as cover it, evened out.
+__host__ __device__ inline int chunk_size(int ctx, int most) {
+  const int n = (ctx + most - 1) / most, even = (ctx + n - 1) / n;
+  return (even + 63) / 64 * 64;
+}
+
+template <typename E>
+struct Geo;
+template <>
+struct Geo<int8_t> {
+  static constexpr int KT = 64, PL = 1;  // tokens of a context tile, fp16 pieces of K and V
+};
+template <>
+struct Geo<float> {
+  static constexpr int KT = 32, PL = 2;
+};
+
+// Scheduling of a chain of N steps that read PL fragments from LDS and run M products each: the
+// reads go kAhead steps before their products (left to itself the compiler reads a fragment right
+// before them and waits out the LDS latency at every step).
+template <int N, int PL, int M>
+__device__ __forceinline__ void read_ahead() {
+  constexpr int kAhead = 2, kRead = 0x100, kMfma = 0x8;
+  __builtin_amdgcn_sched_group_barrier(kRead, kAhead * PL, 0);
+#pragma unroll
+  for (int i = 0; i < N - kAhead; ++i) {
+    __builtin_amdgcn_sched_group_barrier(kMfma, M, 0);
+    __builtin_amdgcn_sched_group_barrier(kRead, PL, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(kMfma, kAhead * M, 0);
+}
+
+template <typename E, int D>
+__global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a) {
+  constexpr bool kF32 = std::is_same_v<E, float>;
+  constexpr int KT = Geo<E>::KT, PL = Geo<E>::PL;
+  constexpr int TT = KT / 16;   // 16-token tiles of a context tile
+  constexpr int KS = D / 32;    // MFMA steps of q . k
+  constexpr int DT = D / 16;    // 16-dim tiles of the output
+  constexpr int VS = KT / 32;   // MFMA steps of p v
+  constexpr int kKBytes = PL * TT * KS * kFrag, kVBytes = PL * DT * VS * kFrag;
+  constexpr int TW = KT / kWaves;                           // context tokens a wavefront stages
+  constexpr int kRow = D * static_cast<int>(sizeof(E));     // bytes of a cache row
+  constexpr int kLoads = TW * kRow / kFrag;                 // 1 KB loads of a wavefront, K or V
+  __shared__ __attribute__((aligned(16))) char conv[kKBytes + kVBytes];            // fp16 fragments
+  __shared__ __attribute__((aligned(16))) char raw[kWaves][2][kLoads * kFrag];     // rows as cached
+  __shared__ __attribute__((aligned(16))) float sk[KT], sv[KT];                    // the tokens' scales
+  __shared__ uint32_t have[kWaves];                                                // bits: the tokens that exist
+
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int fr = lane % 16, fc = lane / 16;
+  const int hp = blockIdx.x, kvh = hp / a.pairs, g0 = hp % a.pairs * kHeads;
+  const int tile = blockIdx.y, chunk = blockIdx.z;
+  const int row0 = static_cast<int>(a.tiles[4 * tile]), rows = static_cast<int>(a.tiles[4 * tile + 1]);
+  const int sees = static_cast<int>(a.tiles[4 * tile + 2]), tab = static_cast<int>(a.tiles[4 * tile + 3]);
+  const int ctx = sees + rows - 1;  // tokens the tile's last row sees
+  const int size = chunk_size(ctx, a.chunk), k0 = chunk * size;
+  if (k0 >= ctx) return;  // whole workgroup
+  const int k1 = min(ctx, k0 + size);
+  const int n_ct = (k1 - k0 + KT - 1) / KT;
+
+  // ---- q: this wavefront's 16 tokens, both heads, as B operands --------------------------------
+  const int tok = min(16 * wave + fr, rows - 1);
+  int head[kHeads];
+  f16x8 qf[kHeads][KS][2];
+  float qs[kHeads];  // score = dot * k_scale * qs (log2 units)
+#pragma unroll
+  for (int c = 0; c < kHeads; ++c) {
+    head[c] = kvh * a.G + min(g0 + c, a.G - 1);
+    const float* qp = a.q + (static_cast<int64_t>(row0 + tok) * a.Hq + head[c]) * D + 8 * fc;
+    float v[KS][8];
+    float top = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(qp + 32 * s);
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(qp + 32 * s + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[s][e] = lo[e];
+        v[s][4 + e] = hi[e];
+      }
+      if (a.q_mult) {
+        const float* mp = a.q_mult + head[c] * D + 32 * s + 8 * fc;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[s][e] = __fmul_rn(v[s][e], mp[e]);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(v[s][e]));
+    }
+    const int ex = exponent_to_15(max_over_fc(top));
+    // the sign of the softmax scale goes with q, so that qs >= 0 and the scores' order is the dots'
+    const float up = __builtin_copysignf(__builtin_amdgcn_ldexpf(1.f, ex), a.scale);
+    qs[c] = fmaxf(__builtin_amdgcn_ldexpf(fabsf(a.scale) * kLog2e, -ex), 1e-37f);  // 0: -inf * 0 below
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      u32x4 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t h, l;
+        split2(v[s][2 * e] * up, v[s][2 * e + 1] * up, h, l);
+        hi[e] = h;
+        lo[e] = l;
+      }
+      qf[c][s][0] = __builtin_bit_cast(f16x8, hi);
+      qf[c][s][1] = __builtin_bit_cast(f16x8, lo);
+    }
+  }
+
+  // ---- staging: wavefront w brings tokens TW w .. + TW of a context tile ------------------------
+  // block id of the token this lane looks after (lane % TW of the wavefront's), read a tile ahead
+  const int64_t* bt = a.bt + static_cast<int64_t>(tab) * a.max_blocks;
+  auto token_of = [&](int it) { return k0 + it * KT + TW * wave + lane % TW; };
+  auto block_of = [&](int t) { return a.bs_shift >= 0 ? t >> a.bs_shift : t / a.bs; };
+  auto fetch_id = [&](int it) {
+    const int t = token_of(it);
+    return t < k1 ? bt[block_of(t)] : static_cast<int64_t>(-1);
+  };
+  const int64_t blocks = a.num_slots / a.bs, rstride = static_cast<int64_t>(a.Hk) * kRow;
+  auto slot_of = [&](int it, int64_t id) {  // cache slot, -1: no such token
+    const int t = token_of(it);
+    return id < 0 || id >= blocks ? -1 : static_cast<int>(id) * a.bs + (t - block_of(t) * a.bs);
+  };
+  // starts the loads of a tile's rows (straight into LDS) and of this lane's scale
+  float scale = 0.f;
+  auto load = [&](int slot) {
+    constexpr int kTok = kFrag / kRow;  // tokens of a load
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int s = __shfl(slot, i * kTok + lane / (kWave / kTok), kWave);
+      const int64_t at = (s < 0 ? 0 : s) * rstride + kvh * kRow + lane % (kWave / kTok) * 16;
+      __builtin_amdgcn_global_load_lds(static_cast<const char*>(a.kc) + at,
+                                       (__attribute__((address_space(3))) void*)(raw[wave][0] + i * kFrag), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(static_cast<const char*>(a.vc) + at,
+                                       (__attribute__((address_space(3))) void*)(raw[wave][1] + i * kFrag), 16, 0, 0);
+    }
+    if constexpr (!kF32) {  // lanes 0 .. TW - 1 K scales, the next TW V scales
+      const float* p = lane < TW ? a.ks : a.vs;
+      scale = slot >= 0 ? p[static_cast<int64_t>(slot) * a.Hk + kvh] : 0.f;
+    }
+  };
+  // V: 4 tokens x VD dims per thread, transposed into [dim][token] on the way
+  constexpr int VD = kF32 ? 4 : D / 16;
+  constexpr int kVLanes = D / VD;
+  const bool v_on = TW / 4 * kVLanes == kWave || lane < TW / 4 * kVLanes;
+  const int vd0 = lane % kVLanes * VD, vl0 = lane / kVLanes % (TW / 4) * 4;  // dims, token of the wavefront's
+  const int vg = TW / 4 * wave + vl0 / 4;                                    // group of 4 tokens in the tile
+  // chunk c (8 dims) of token t: fragment (t / 16, c / 4), lane position t % 16 moved by `swz` so
+  // that the writes of a row's lanes fall into different banks
+  auto swz = [](int c) { return kF32 ? c & 7 : (c >> 1) * (128 / D); };
+  auto k_at = [&](char* base, int pl, int t, int c) {
+    return base + ((pl * TT + t / 16) * KS + c / 4) * kFrag + (((t % 16) ^ swz(c)) + 16 * (c % 4)) * 16;
+  };
+  // dim d, tokens 4 g .. + 3: fragment (d / 16, token / 32), lane d % 16 + 16 (g % 4), its first or
+  // second four elements for the even or odd 16-token tile
+  auto v_at = [&](char* base, int pl, int d, int g) {
+    return base + kKBytes + ((pl * DT + d / 16) * VS + g / 8) * kFrag +
+           (((d % 16) ^ (d / 16 % 8)) + 16 * (g % 4)) * 16 + g / 4 % 2 * 8;
+  };
+  // this wavefront's landed rows -> fragments; `slot` as for their load
+  auto convert = [&](int slot) {
+    const uint64_t ok = __ballot(slot >= 0);
+    if (lane == 0) have[wave] = static_cast<uint32_t>(ok) & ((1u << TW) - 1);
+    if constexpr (!kF32) {
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) {
+        const int j = i * kWave + lane, t = TW * wave + j * 16 / kRow, c = j * 16 % kRow / 8;
+        const u32x4 r = *reinterpret_cast<const u32x4*>(raw[wave][0] + j * 16);
+        u32x4 lo, hi;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          const uint32_t x = r[w] ^ 0x80808080u, y = r[2 + w] ^ 0x80808080u;
+          lo[2 * w] = bytes_to_h2<0x04010400u>(x);
+          lo[2 * w + 1] = bytes_to_h2<0x04030402u>(x);
+          hi[2 * w] = bytes_to_h2<0x04010400u>(y);
+          hi[2 * w + 1] = bytes_to_h2<0x04030402u>(y);
+        }
+        *reinterpret_cast<u32x4*>(k_at(conv, 0, t, c)) = lo;
+        *reinterpret_cast<u32x4*>(k_at(conv, 0, t, c + 1)) = hi;
+      }
+#pragma unroll
+      for (int w = 0; w < VD / 4; ++w) {
+        uint32_t x[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          x[t] = *reinterpret_cast<const uint32_t*>(raw[wave][1] + (vl0 + t) * kRow + vd0 + 4 * w) ^ 0x80808080u;
+        // bytes of tokens (0, 1) and (2, 3) side by side: [a0 b0 a1 b1], [a2 b2 a3 b3]
+        const uint32_t p01 = __builtin_amdgcn_perm(x[1], x[0], 0x05010400u), p23 = __builtin_amdgcn_perm(x[3], x[2], 0x05010400u);
+        const uint32_t q01 = __builtin_amdgcn_perm(x[1], x[0], 0x07030602u), q23 = __builtin_amdgcn_perm(x[3], x[2], 0x07030602u);
+        const int d = vd0 + 4 * w;
+        *reinterpret_cast<u32x2*>(v_at(conv, 0, d, vg)) = u32x2{bytes_to_h2<0x04010400u>(p01), bytes_to_h2<0x04010400u>(p23)};
+        *reinterpret_cast<u32x2*>(v_at(conv, 0, d + 1, vg)) = u32x2{bytes_to_h2<0x04030402u>(p01), bytes_to_h2<0x04030402u>(p23)};
+        *reinterpret_cast<u32x2*>(v_at(conv, 0, d + 2, vg)) = u32x2{bytes_to_h2<0x04010400u>(q01), bytes_to_h2<0x04010400u>(q23)};
+        *reinterpret_cast<u32x2*>(v_at(conv, 0, d + 3, vg)) = u32x2{bytes_to_h2<0x04030402u>(q01), bytes_to_h2<0x04030402u>(q23)};
+      }
+      if (lane < TW) sk[TW * wave + lane] = scale;
+      if (lane >= TW && lane < 2 * TW) sv[TW * wave + lane - TW] = fminf(scale * kUp, kHuge);
+    } else {
+      // a row's exponent, from the largest magnitude as an integer (NaN and infinity above all)
+      auto row_scale = [&](uint32_t top, int lanes, float& up) {
+        for (int m = 1; m < lanes; m <<= 1) {
+          const uint32_t o = static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), m, kWave));
+          top = top > o ? top : o;
+        }
+        const int ex = exponent_to_15(__builtin_bit_cast(float, top));
+        const bool bad = top >= 0x7f800000u;  // the row reads as zeros, its scale as not finite
+        up = bad ? 0.f : __builtin_amdgcn_ldexpf(1.f, ex);
+        return bad ? __builtin_nanf("") : __builtin_amdgcn_ldexpf(1.f, -ex);
+      };
+      auto mag = [](const u32x4& w) {
+        uint32_t t = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t b = w[e] & 0x7fffffffu;
+          t = t > b ? t : b;
+        }
+        return t;
+      };
+      auto value = [](const u32x4& w, int e, float up) {
+        const uint32_t u = w[e];
+        return up == 0.f ? 0.f : __builtin_bit_cast(float, u) * up;
+      };
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) {
+        const int j = i * kWave + lane, tl = j * 16 / kRow, t = TW * wave + tl, p = j * 16 % kRow / 16;
+        const u32x4 r = *reinterpret_cast<const u32x4*>(raw[wave][0] + j * 16);
+        float up;
+        const float down = row_scale(mag(r), kRow / 16, up);
+        uint32_t h0, l0, h1, l1;
+        split2(value(r, 0, up), value(r, 1, up), h0, l0);
+        split2(value(r, 2, up), value(r, 3, up), h1, l1);
+        *reinterpret_cast<u32x2*>(k_at(conv, 0, t, p / 2) + p % 2 * 8) = u32x2{h0, h1};
+        *reinterpret_cast<u32x2*>(k_at(conv, 1, t, p / 2) + p % 2 * 8) = u32x2{l0, l1};
+        if (p == 0) sk[t] = ok >> tl & 1 ? down : 0.f;
+      }
+      u32x4 r[4];
+      float up[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        r[t] = *reinterpret_cast<const u32x4*>(raw[wave][1] + (vl0 + t) * kRow + vd0 * 4);
+        const float down = row_scale(mag(r[t]), kVLanes, up[t]);
+        if (v_on && vd0 == 0) sv[4 * vg + t] = ok >> (vl0 + t) & 1 ? fminf(down * kUp, kHuge) : 0.f;
+      }
+      if (v_on) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          uint32_t h0, l0, h1, l1;
+          split2(value(r[0], e, up[0]), value(r[1], e, up[1]), h0, l0);
+          split2(value(r[2], e, up[2]), value(r[3], e, up[3]), h1, l1);
+          *reinterpret_cast<u32x2*>(v_at(conv, 0, vd0 + e, vg)) = u32x2{h0, h1};
+          *reinterpret_cast<u32x2*>(v_at(conv, 1, vd0 + e, vg)) = u32x2{l0, l1};
+        }
+      }
+    }
+  };
+
+  // ---- the context ------------------------------------------------------------------------------
+  f32x4 acc[kHeads][DT];
+  float ref[kHeads], sum[kHeads];
+#pragma unroll
+  for (int c = 0; c < kHeads; ++c) {
+    ref[c] = -1e30f;
+    sum[c] = 0.f;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) acc[c][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const int limit = sees + tok;  // tokens this lane's query sees
+
+  int slot = slot_of(0, fetch_id(0));
+  load(slot);
+  int64_t id = fetch_id(1);
+  for (int it = 0; it < n_ct; ++it) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's rows have landed
+    if (it) __syncthreads();             // everyone has read the last tile's fragments
+    convert(slot);
+    if (it + 1 < n_ct) {  // the rows are read (their values are in use): the next ones may land
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      slot = slot_of(it + 1, id);
+      load(slot);
+      id = fetch_id(it + 2);
+    }
+    __syncthreads();
+    const char* base = conv;
+    __builtin_amdgcn_s_setprio(1);
+    f32x4 s[kHeads][TT];
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+      // Two sums per score, added at the end: the first half of the hi products in one, the rest, with
+      // the small products of lo pieces, in the other. One chain would round at the score's size three
+      // times as often: measured error against float64 2.1e-7 with one, 1.7e-7 with two (int8, 1000
+      // tokens); more than two change nothing.
+      f32x4 part[kHeads][2] = {};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int c = 4 * ks + fc, half = 2 * ks / KS;
+        const char* p = base + (tt * KS + ks) * kFrag + ((fr ^ swz(c)) + 16 * fc) * 16;
+        f16x8 kf[PL];
+#pragma unroll
+        for (int pl = 0; pl < PL; ++pl)
+          kf[pl] = *reinterpret_cast<const f16x8*>(p + pl * TT * KS * kFrag);
+#pragma unroll
+        for (int c2 = 0; c2 < kHeads; ++c2) part[c2][1] = mfma(kf[0], qf[c2][ks][1], part[c2][1]);
+        if constexpr (PL == 2) {
+#pragma unroll
+          for (int c2 = 0; c2 < kHeads; ++c2) part[c2][1] = mfma(kf[1], qf[c2][ks][0], part[c2][1]);
+        }
+#pragma unroll
+        for (int c2 = 0; c2 < kHeads; ++c2) part[c2][half] = mfma(kf[0], qf[c2][ks][0], part[c2][half]);
+      }
+#pragma unroll
+      for (int c2 = 0; c2 < kHeads; ++c2) s[c2][tt] = part[c2][0] + part[c2][1];
+    }
+    read_ahead<TT * KS, PL, kHeads * (PL + 1)>();
+    __builtin_amdgcn_s_setprio(0);
+    // scores (times qs: log2 units); lane (fr, fc) holds tokens 16 tt + 4 fc + e of its query
+    float vtop = 0.f;  // the largest v scale
+    const int t0 = k0 + it * KT;
+    uint64_t there = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) there |= static_cast<uint64_t>(have[w]) << (TW * w);
+    const bool hole = t0 + KT > sees + min(16 * wave, rows - 1) ||  // some lane's query ends in this tile
+                      there != (KT == 64 ? ~0ull : (1ull << KT) - 1);
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+      const f32x4 kk = *reinterpret_cast<const f32x4*>(&sk[16 * tt + 4 * fc]);
+      const f32x4 vv = *reinterpret_cast<const f32x4*>(&sv[16 * tt + 4 * fc]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        vtop = fmaxf(vtop, vv[e]);
+#pragma unroll
+        for (int c = 0; c < kHeads; ++c) s[c][tt][e] *= kk[e];
+      }
+    }
+    if (hole) {  // (the largest v scale, too, of the tokens this lane's query sees)
+      vtop = 0.f;
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        const f32x4 vv = *reinterpret_cast<const f32x4*>(&sv[16 * tt + 4 * fc]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = 4 * fc + e;
+          const bool in = t0 + 16 * tt + t < limit && (static_cast<uint32_t>(there >> (16 * tt)) >> t & 1);
+          vtop = fmaxf(vtop, in ? vv[e] : 0.f);
+#pragma unroll
+          for (int c = 0; c < kHeads; ++c) s[c][tt][e] = in ? s[c][tt][e] : -__builtin_inff();
+        }
+      }
+    }
+    const float lv = fminf(fmaxf(__builtin_amdgcn_logf(max_over_fc(vtop) * (1.f / kUp)), -kMaxLv), kMaxLv);
+    float top[kHeads];
+    bool raise = false;
+#pragma unroll
+    for (int c = 0; c < kHeads; ++c) {
+      top[c] = s[c][0][0];
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) top[c] = fmaxf(top[c], s[c][tt][e]);
+      top[c] *= qs[c];
+      raise |= top[c] + lv > ref[c] + kLazy;
+    }
+    if (__ballot(raise) != 0) {
+#pragma unroll
+      for (int c = 0; c < kHeads; ++c) {
+        const float want = max_over_fc(top[c]) + lv;
+        const float now = want > ref[c] + kLazy ? want : ref[c];
+        const float f = __builtin_amdgcn_exp2f(ref[c] - now);
+        ref[c] = now;
+        sum[c] *= f;
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[c][d][e] *= f;
+      }
+    }
+    // weights and their product with V
+#pragma unroll
+    for (int vs = 0; vs < VS; ++vs) {
+      f16x8 ph[kHeads], pl[kHeads];
+      f32x4 vsc[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        vsc[h] = *reinterpret_cast<const f32x4*>(&sv[16 * (2 * vs + h) + 4 * fc]);
+#pragma unroll
+      for (int c = 0; c < kHeads; ++c) {
+        u32x4 hi, lo;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float w[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[c][2 * vs + h][e], qs[c], -ref[c]));
+            sum[c] += p;
+            w[e] = p * vsc[h][e];
+          }
+          uint32_t h0, l0, h1, l1;
+          split2(w[0], w[1], h0, l0);
+          split2(w[2], w[3], h1, l1);
+          hi[2 * h] = h0;
+          hi[2 * h + 1] = h1;
+          lo[2 * h] = l0;
+          lo[2 * h + 1] = l1;
+        }
+        ph[c] = __builtin_bit_cast(f16x8, hi);
+        pl[c] = __builtin_bit_cast(f16x8, lo);
+      }
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        const char* p = base + kKBytes + (d * VS + vs) * kFrag + ((fr ^ (d % 8)) + 16 * fc) * 16;
+        f16x8 vf[PL];
+#pragma unroll
+        for (int q = 0; q < PL; ++q) vf[q] = *reinterpret_cast<const f16x8*>(p + q * DT * VS * kFrag);
+if constexpr (PL == 1) {
+#pragma unroll
+          for (int c = 0; c < kHeads; ++c) acc[c][d] = mfma(vf[0], ph[c], acc[c][d]);
+#pragma unroll
+          for (int c = 0; c < kHeads; ++c) acc[c][d] = mfma(vf[0], pl[c], acc[c][d]);
+        } else {  // the tile's sum apart, its small products first: one rounding at acc's size
+          f32x4 t[kHeads];
+#pragma unroll
+          for (int c = 0; c < kHeads; ++c) t[c] = mfma(vf[PL - 1], ph[c], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+          for (int c = 0; c < kHeads; ++c) t[c] = mfma(vf[0], pl[c], t[c]);
+#pragma unroll
+          for (int c = 0; c < kHeads; ++c) acc[c][d] += mfma(vf[0], ph[c], t[c]);
+        }
+      }
+      __builtin_amdgcn_s_setprio(0);
+    }
+  }
+
+  // ---- output: lane (fr, fc) holds dims 16 d + 4 fc + e of its query -----------------------------
+  const bool whole = size >= ctx;
+#pragma unroll
+  for (int c = 0; c < kHeads; ++c) {
+    const float l = sum_over_fc(sum[c]);
+    if (16 * wave + fr >= rows || g0 + c >= a.G) continue;
+    if (whole) {
+      const float inv = 1.f / (l * kUp);
+      float* o = a.out + (static_cast<int64_t>(row0 + tok) * a.Hq + head[c]) * D + 4 * fc;
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+        *reinterpret_cast<f32x4*>(o + 16 * d) = acc[c][d] * inv;
+    } else {
+      const int64_t at = (((static_cast<int64_t>(tile) * a.Hk * a.pairs + hp) * a.splits + chunk) * kHeads + c) * kQT + tok;
+      float* o = a.part_acc + at * D + 4 * fc;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4*>(o + 16 * d) = acc[c][d];
+      if (fc == 0) {
+        a.part_rl[2 * at] = ref[c];
+        a.part_rl[2 * at + 1] = l;
+      }
+    }
+  }
+}
+
+// Adds the chunks of the tiles that have several: one wavefront per (tile, query token, head).
+//   R = max_j r_j;  out = sum_j 2^(r_j - R) acc_j / sum_j 2^(r_j - R) l_j   (l_j = 0 skipped)
+template <int D>
+__global__ __launch_bounds__(kWaves* kWave) void prefill_merge_kernel(PrefillArgs a) {
+  constexpr int PER = D / kWave;
+  const int tile = blockIdx.y, lane = threadIdx.x % kWave;
+  const int rows = static_cast<int>(a.tiles[4 * tile + 1]);
+  const int ctx = static_cast<int>(a.tiles[4 * tile + 2]) + rows - 1, size = chunk_size(ctx, a.chunk);
+  const int n = (ctx + size - 1) / size;
+  const int i = blockIdx.x * kWaves + threadIdx.x / kWave, tok = i / a.Hq, h = i % a.Hq;
+  if (n <= 1 || tok >= rows) return;
+  const int kvh = h / a.G, g = h % a.G, hp = kvh * a.pairs + g / kHeads, c = g % kHeads;
+  const int64_t base = ((static_cast<int64_t>(tile) * a.Hk * a.pairs + hp) * a.splits * kHeads + c) * kQT + tok;
+  const int64_t step = static_cast<int64_t>(kHeads) * kQT;
+  float R = -1e30f;
+  for (int j = 0; j < n; ++j) R = fmaxf(R, a.part_rl[2 * (base + j * step)]);
+  float L = 0.f, o[PER] = {};
+  for (int j = 0; j < n; ++j) {
+    const float l = a.part_rl[2 * (base + j * step) + 1];
+    const float w = l == 0.f ? 0.f : __builtin_amdgcn_exp2f(a.part_rl[2 * (base + j * step)] - R);
+    L += w * l;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) o[e] += w * a.part_acc[(base + j * step) * D + lane * PER + e];
+  }
+  const float inv = 1.f / (L * kUp);
+  float* out = a.out + (static_cast<int64_t>(a.tiles[4 * tile] + tok) * a.Hq + h) * D + lane * PER;
+#pragma unroll
+  for (int e = 0; e < PER; ++e) out[e] = o[e] * inv;
+}
+
+int device_cus() {
+  int dev = 0, c = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0)
+    return 256;
+  return c;
+}
+
+struct ChunkPlan {
+  int chunk, splits;  // chunk tokens (a multiple of 64), most chunks of a tile
+};
+
+// The chunk size by an estimate in context tiles of 64 tokens: a launch of at most two workgroups per
+// CU takes as long as its longest chunk, a larger one its share of the work and half of that; one
+// workgroup per CU runs a tile in 3.2 us, two side by side in 4.8 (2048 tokens, one launch of each);
+// the merge of the chunks costs about 3 tiles. 2048 new tokens, 16 / 8 heads: 115 us in one chunk,
+// 73 at 704 tokens, 83 at 576 (a few workgroups start a second round).
+ChunkPlan plan_chunks(const int64_t* tiles, int64_t n, int64_t groups) {
+  int64_t total = 0, longest = 1;
+  for (int64_t i = 0; i < n; ++i) {
+    const int64_t t = (tiles[4 * i + 1] + tiles[4 * i + 2] - 1 + 63) / 64;
+    total += t;
+    longest = std::max(longest, t);
+  }
+  const int64_t cus = device_cus(), slots = 2 * cus;
+  auto cost = [&](int64_t units, int64_t len, bool merge) {
+    const double one = units <= cus ? 0.67 : 1.0;
+    return (units <= slots ? one * len : static_cast<double>(total * groups) / slots + 0.5 * len) + (merge ? 3.0 : 0.0);
+  };
+  double best = cost(n * groups, longest, false);
+  int64_t take = longest;
+  if (n * groups < 4 * slots) {
+    const int64_t step = std::max<int64_t>(1, longest / 48);
+    for (int64_t c = 4; c < longest; c += step) {
+      int64_t units = 0, len = 1;
+      for (int64_t i = 0; i < n; ++i) {
+        const int64_t t = (tiles[4 * i + 1] + tiles[4 * i + 2] - 1 + 63) / 64, k = (t + c - 1) / c;
+        units += k;
+        len = std::max(len, (t + k - 1) / k);
+      }
+      const double v = cost(units * groups, len, true);
+      if (v < best) {
+        best = v;
+        take = c;
+      }
+    }
+  }
+  return {static_cast<int>(take * 64), static_cast<int>((longest + take - 1) / take)};
+}
+
+int64_t partial_floats(int64_t n, int64_t groups, int64_t splits, int64_t D) {
+  return splits > 1 ? n * groups * splits * kHeads * kQT * (D + 2) : 0;
+}
+
+int64_t head_pairs(int64_t Hq, int64_t Hk) { return Hk * ((Hq / Hk + kHeads - 1) / kHeads); }
+
+}  // namespace
+
+extern "C" int64_t llmserve_paged_attention_prefill_workspace_bytes(const int64_t* tiles_host, int64_t n_tiles,
+                                                                    int64_t Hq, int64_t Hk, int64_t D) {
+  if (n_tiles <= 0 || Hq <= 0 || Hk <= 0 || Hq % Hk || tiles_host == nullptr) return 0;
+  const int64_t groups = head_pairs(Hq, Hk);
+  return partial_floats(n_tiles, groups, plan_chunks(tiles_host, n_tiles, groups).splits, D) * 4;
+}
+
+extern "C" int llmserve_paged_attention_prefill(const float* q, const void* k_cache, const void* v_cache,
+                                                const float* k_scale, const float* v_scale,
+                                                const int64_t* block_tables, int64_t table_rows,
+                                                const int64_t* tiles, const int64_t* tiles_host, int64_t n_tiles,
+                                                float* out, int64_t T, int64_t Hq, int64_t Hk, int64_t D,
+                                                int64_t num_slots, int64_t max_blocks, int64_t block_size,
+                                                float scale, const float* q_mult, void* workspace,
+                                                int64_t workspace_bytes, void* stream) {
+  LSH_CHECK(T >= 0 && Hq >= 1 && Hk >= 1 && Hq % Hk == 0 && n_tiles >= 0, "paged_attention_prefill: bad shape");
+  LSH_CHECK(D == 64 || D == 128, "paged_attention_prefill: head_dim %lld not 64 or 128", (long long)D);
+  if (n_tiles == 0) return LLMSERVE_OK;
+  LSH_CHECK(block_size >= 1 && max_blocks >= 1 && num_slots >= block_size && table_rows >= 1,
+            "paged_attention_prefill: empty block table or cache");
+  LSH_CHECK(max_blocks * block_size < (1LL << 30) && num_slots * Hk < (1LL << 31) && T < (1LL << 24) && Hk <= 4096 &&
+                Hq <= 32768 && n_tiles < 65536,
+            "paged_attention_prefill: batch, context or cache too large");
+  LSH_CHECK(q && k_cache && v_cache && block_tables && tiles && tiles_host && out && (!k_scale == !v_scale),
+            "paged_attention_prefill: null pointer");
+  LSH_CHECK(lsh::aligned16(q) && lsh::aligned16(k_cache) && lsh::aligned16(v_cache) && lsh::aligned16(out),
+            "paged_attention_prefill: q, caches and out must be 16-byte aligned");
+  for (int64_t i = 0; i < n_tiles; ++i) {
+    const int64_t* t = tiles_host + 4 * i;
+    LSH_CHECK(t[0] >= 0 && t[1] >= 1 && t[1] <= kQT && t[0] + t[1] <= T && t[2] >= 1 &&
+                  t[2] + t[1] - 1 <= max_blocks * block_size && t[3] >= 0 && t[3] < table_rows,
+              "paged_attention_prefill: tile %lld outside the batch or its block table", (long long)i);
+  }
+  PrefillArgs a{};
+  a.G = static_cast<int>(Hq / Hk);
+  a.pairs = (a.G + kHeads - 1) / kHeads;
+  const int64_t groups = Hk * a.pairs;
+  const ChunkPlan plan = plan_chunks(tiles_host, n_tiles, groups);
+  const int64_t floats = partial_floats(n_tiles, groups, plan.splits, D);
+  LSH_CHECK(floats == 0 || (workspace != nullptr && workspace_bytes >= floats * 4 && lsh::aligned16(workspace)),
+            "paged_attention_prefill: a 16-byte aligned workspace of %lld bytes is needed (%lld given)",
+            (long long)(floats * 4), (long long)workspace_bytes);
+  a.q = q;
+  a.kc = k_cache;
+  a.vc = v_cache;
+  a.ks = k_scale;
+  a.vs = v_scale;
+  a.bt = block_tables;
+  a.tiles = tiles;
+  a.q_mult = q_mult;
+  a.out = out;
+  a.part_acc = static_cast<float*>(workspace);
+  a.part_rl = a.part_acc + floats / (D + 2) * D;
+  a.num_slots = num_slots;
+  a.n_tiles = static_cast<int>(n_tiles);
+  a.Hq = static_cast<int>(Hq);
+  a.Hk = static_cast<int>(Hk);
+  a.max_blocks = static_cast<int>(max_blocks);
+  a.bs = static_cast<int>(block_size);
+  a.bs_shift = -1;
+  for (int sh = 0; sh < 30; ++sh)
+    if ((1LL << sh) == block_size) a.bs_shift = sh;
+  a.chunk = plan.chunk;
+  a.splits = plan.splits;
+  a.scale = scale;
+  hipStream_t st = lsh::as_stream(stream);
+  const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(n_tiles), static_cast<unsigned>(plan.splits));
+  const dim3 block(kWaves * kWave);
+  const bool once = plan.splits == 1;
+  if (k_scale != nullptr && D == 128)
+    lsh::launch(prefill_kernel<int8_t, 128>, grid, block, 0, st, once, a);
+  else if (k_scale != nullptr)
+    lsh::launch(prefill_kernel<int8_t, 64>, grid, block, 0, st, once, a);
+  else if (D == 128)
+    lsh::launch(prefill_kernel<float, 128>, grid, block, 0, st, once, a);
+  else
+    lsh::launch(prefill_kernel<float, 64>, grid, block, 0, st, once, a);
+  if (!once) {
+    const dim3 mgrid(static_cast<unsigned>(kQT * Hq / kWaves), static_cast<unsigned>(n_tiles));
+    if (D == 128)
+      lsh::launch(prefill_merge_kernel<128>, mgrid, block, 0, st, true, a);
+    else
+      lsh::launch(prefill_merge_kernel<64>, mgrid, block, 0, st, true, a);
+  }
+  return lsh::launch_status("paged_attention_prefill");
+}

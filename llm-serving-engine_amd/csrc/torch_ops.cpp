@@ -840,6 +840,60 @@ at::Tensor paged_attention_rows(const at::Tensor& q, const at::Tensor& k_cache,
   return out;
 }
 
+// The rows of `out` that the tiles cover; tiles_host holds the values of tiles (both int64 [n, 4]).
+void paged_attention_prefill_(at::Tensor out, const at::Tensor& q, const at::Tensor& k_cache,
+                              const at::Tensor& v_cache, const std::optional<at::Tensor>& k_scale,
+                              const std::optional<at::Tensor>& v_scale, const at::Tensor& block_tables,
+                              const at::Tensor& tiles, const at::Tensor& tiles_host, int64_t block_size,
+                              double scale, const std::optional<at::Tensor>& q_mult) {
+  const char* what = "paged_attention_prefill_";
+  const bool int8 = k_cache.scalar_type() == at::kChar;
+  TORCH_CHECK(int8 || k_cache.scalar_type() == at::kFloat, what, ": int8 or float32 cache");
+  TORCH_CHECK(v_cache.scalar_type() == k_cache.scalar_type() && v_cache.sizes() == k_cache.sizes(), what,
+              ": K and V caches of one type and shape");
+  TORCH_CHECK(int8 == (k_scale.has_value() && v_scale.has_value()), what,
+              ": an int8 cache takes k_scale and v_scale, a float32 one none");
+  TORCH_CHECK(q.scalar_type() == at::kFloat && q.dim() == 3 && q.is_contiguous() &&
+                  out.scalar_type() == at::kFloat && out.sizes() == q.sizes() && out.is_contiguous(),
+              what, ": q and out must be contiguous float32 [T, Hq, D] tensors");
+  TORCH_CHECK(k_cache.dim() == 3 && k_cache.size(2) == q.size(2) && k_cache.is_contiguous() &&
+                  v_cache.is_contiguous(),
+              what, ": caches must be contiguous [num_slots, Hk, D]");
+  TORCH_CHECK(block_tables.scalar_type() == at::kLong && block_tables.dim() == 2 && block_tables.is_contiguous(),
+              what, ": int64 contiguous block tables");
+  for (const at::Tensor* t : {&tiles, &tiles_host})
+    TORCH_CHECK(t->scalar_type() == at::kLong && t->is_contiguous() && t->dim() == 2 && t->size(1) == 4, what,
+                ": int64 contiguous tiles [n, 4]");
+  TORCH_CHECK(tiles_host.is_cpu() && tiles_host.size(0) == tiles.size(0), what,
+              ": tiles_host must hold the values of tiles on the CPU");
+  check_device(q, {&out, &k_cache, &v_cache, &block_tables, &tiles}, what);
+  const int64_t T = q.size(0), Hq = q.size(1), D = q.size(2);
+  const int64_t num_slots = k_cache.size(0), Hk = k_cache.size(1), n = tiles.size(0);
+  if (int8) {
+    check_device(q, {&*k_scale, &*v_scale}, what);
+    TORCH_CHECK(k_scale->scalar_type() == at::kFloat && v_scale->scalar_type() == at::kFloat &&
+                    k_scale->is_contiguous() && v_scale->is_contiguous() &&
+                    k_scale->numel() == num_slots * Hk && v_scale->numel() == num_slots * Hk,
+                what, ": float32 contiguous scales [num_slots, Hk]");
+  }
+  if (q_mult.has_value()) {
+    check_device(q, {&*q_mult}, what);
+    TORCH_CHECK(q_mult->scalar_type() == at::kFloat && q_mult->is_contiguous() && q_mult->numel() == Hq * D, what,
+                ": q_mult must be a contiguous float32 [Hq, D] tensor");
+  }
+  const c10::DeviceGuard guard(q.device());
+  const int64_t* host = tiles_host.data_ptr<int64_t>();
+  const int64_t ws_bytes = llmserve_paged_attention_prefill_workspace_bytes(host, n, Hq, Hk, D);
+  at::Tensor ws;
+  if (ws_bytes > 0) ws = at::empty({ws_bytes}, q.options().dtype(at::kByte));
+  check_status(llmserve_paged_attention_prefill(
+      q.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(), opt_ptr<float>(k_scale),
+      opt_ptr<float>(v_scale), block_tables.data_ptr<int64_t>(), block_tables.size(0),
+      tiles.data_ptr<int64_t>(), host, n, out.data_ptr<float>(), T, Hq, Hk, D, num_slots,
+      block_tables.size(1), block_size, static_cast<float>(scale), opt_ptr<float>(q_mult),
+      ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(q)));
+}
+
 std::tuple<at::Tensor, at::Tensor, at::Tensor> attention_metadata(const at::Tensor& seq_info,
                                                                   const at::Tensor& block_tables,
                                                                   int64_t block_size, int64_t T) {
@@ -914,6 +968,9 @@ TORCH_LIBRARY(llmserve_hip, m) {
   m.def("paged_attention_rows(Tensor q, Tensor k_cache, Tensor v_cache, Tensor? k_scale,"
         " Tensor? v_scale, Tensor block_tables, Tensor row_table, Tensor row_context,"
         " int block_size, float scale, Tensor? q_mult=None) -> Tensor");
+  m.def("paged_attention_prefill_(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor? k_scale,"
+        " Tensor? v_scale, Tensor block_tables, Tensor tiles, Tensor tiles_host, int block_size,"
+        " float scale, Tensor? q_mult=None) -> ()");
   m.def("attention_metadata(Tensor seq_info, Tensor block_tables, int block_size, int T)"
         " -> (Tensor, Tensor, Tensor)");
 }
@@ -947,6 +1004,7 @@ TORCH_LIBRARY_IMPL(llmserve_hip, CUDA, m) {
   m.impl("paged_attention_decode_int8_xfrag", &paged_attention_decode_int8_xfrag);
   m.impl("paged_attention_decode", &paged_attention_decode);
   m.impl("paged_attention_rows", &paged_attention_rows);
+  m.impl("paged_attention_prefill_", &paged_attention_prefill_);
   m.impl("attention_metadata", &attention_metadata);
 }
 

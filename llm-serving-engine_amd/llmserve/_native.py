@@ -103,6 +103,9 @@ C_SIGNATURES: dict[str, tuple[object, list]] = {
         _I32,
         [_P] * 4 + [_I64] + [_P] * 3 + [_I64] * 7 + [_F32, _P, _P, _I64, _P],
     ),
+    "llmserve_paged_attention_prefill_workspace_bytes": (_I64, [_P, _I64, _I64, _I64, _I64]),
+    "llmserve_paged_attention_prefill": (_I32, [_P] * 6 + [_I64] + [_P] * 2 + [_I64, _P] + [_I64] * 7
+                                         + [ctypes.c_float, _P, _P, _I64, _P]),
     "llmserve_attention_metadata": (_I32, [_P, _P] + [_I64] * 4 + [_P] * 4),
     "llmserve_decode_chain_workspace_bytes": (_I64, [_I64, _I64]),
     "llmserve_decode_chain": (

@@ -12,8 +12,9 @@ Two backends, chosen by ``AttentionMetadata.backend``:
   the slot of every new token and its *query row*: the block-table row it attends over and how
   many tokens it sees (its position + 1, the causal mask). ``paged_attention`` then writes the
   new K/V (int8 caches: one quantize-and-scatter kernel per tensor, key smoothing ``k / s``
-  fused) and runs ONE split-context paged attention launch over all T rows, decode and prefill
-  alike, int8 or fp32 cache, with the smoothing product ``q * s`` fused into its q load.
+  fused) and attends: prompt tokens in tiles of 64 on the matrix cores, the other rows (decode
+  tokens, few new tokens, head sizes without a tiled kernel) by the split-context row kernel,
+  int8 or fp32 cache, with the smoothing product ``q * s`` fused into the q loads.
 * ``"torch"``: slots and per-sequence tables are computed with vectorised numpy on the host;
   attention gathers the (dequantized) context rows and calls SDPA, the reference's algorithm
   (attention.py:249-257, :299-306).
@@ -31,6 +32,15 @@ import torch
 import torch.nn.functional as F
 
 NATIVE_BACKENDS = ("hip", "cpp")
+QUERY_TILE = 64  # query tokens of a prefill tile
+# Which tokens go to the prefill kernel: those of sequences with at least TILE_ROWS new ones, where
+# the row kernel's work on them, sum(new * context), at ROW_US per token outweighs what a tiled launch
+# adds: TILE_US, CTX_US per token of the longest context, and REST_US for a row launch of its own
+# when other tokens remain. Measured at 16 / 8 heads, int8 (rows / tiles, us): one sequence of 32 new
+# tokens in 1024: 21 / 24, 64: 29 / 27, 32 in 4096: 43 / 39, 64 in 256: 17 / 20; eight sequences of 4 in
+# 4096: 47 / 62, of 8: 79 / 61, of 16 in 1024: 50 / 31 (fp32 caches gain from fewer tokens on).
+TILE_ROWS = 8
+ROW_US, TILE_US, CTX_US, REST_US = 0.235e-3, 4.0, 6e-3, 20.0
 
 
 @dataclass
@@ -61,6 +71,14 @@ class AttentionMetadata:
     block_tables: torch.Tensor | None = None  # [S, max_blocks] the batch's tables, zero-padded
     row_table: torch.Tensor | None = None  # [T] the table row token t attends over
     row_context: torch.Tensor | None = None  # [T] how many context tokens token t sees
+    # The tokens of sequences with at least TILE_ROWS new ones, as tiles of the prefill kernel
+    # ([n, 4]: first token, tokens, context the first one sees, table row), on the device and the
+    # host; the other tokens as rows: indices into the batch, table rows, contexts.
+    prefill_tiles: torch.Tensor | None = None
+    prefill_tiles_host: torch.Tensor | None = None
+    rest_rows: torch.Tensor | None = None  # None: every token is in a tile
+    rest_table: torch.Tensor | None = None
+    rest_context: torch.Tensor | None = None
     _prefill_masks: dict[int, torch.Tensor | None] = field(default_factory=dict)
 
     @staticmethod
@@ -148,6 +166,26 @@ class _BatchPlan:
             out.append(PrefillSeq(int(self.q_start[s]), int(self.q[s]), c, slots))
         return out
 
+    def prefill_tiles(self) -> tuple[np.ndarray, np.ndarray]:
+        """(tiles [n, 4], longest context first; the other tokens [3, m]: index, table row,
+        context) for the native backend."""
+        tiled = (self.q >= TILE_ROWS) & (self.ctx >= self.q)
+        seqs = np.flatnonzero(tiled)
+        gain = ROW_US * float((self.q[seqs] * self.ctx[seqs]).sum()) - TILE_US
+        gain -= CTX_US * float(self.ctx[seqs].max(initial=0)) + (REST_US if seqs.size < self.S else 0)
+        if not seqs.size or gain <= 0:
+            return np.zeros((0, 4), np.int64), np.zeros((3, 0), np.int64)
+        tiles = []
+        for s in seqs.tolist():
+            at = np.arange(0, self.q[s], QUERY_TILE)
+            tiles.append(np.stack([self.q_start[s] + at, np.minimum(QUERY_TILE, self.q[s] - at),
+                                   self.ctx[s] - self.q[s] + at + 1, np.full_like(at, s)], axis=1))
+        tiles = np.concatenate(tiles)
+        tiles = np.ascontiguousarray(tiles[np.argsort(-(tiles[:, 1] + tiles[:, 2]), kind="stable")])
+        seq, pos = self.token_positions()
+        rest = np.flatnonzero(~tiled[seq])
+        return tiles, np.stack([rest, seq[rest], pos[rest] + 1])
+
     def fill_host(self, meta: AttentionMetadata, device, native: bool = False) -> None:
         """Everything computed with numpy, then copied to ``device``: the decode rows as
         zero-padded block tables for a native backend (the reference's fields for its kernel),
@@ -172,10 +210,19 @@ class _BatchPlan:
 
     def fill_native(self, meta: AttentionMetadata, device) -> None:
         """Native backend: one upload of the packed batch, then the metadata kernel."""
-        info = np.concatenate([self.q, self.ctx, self.q_start, self.tables.reshape(-1)])
-        dev_info = torch.from_numpy(info).to(device)
+        tiles, rest = self.prefill_tiles()
+        parts = [self.q, self.ctx, self.q_start, self.tables.reshape(-1), tiles.reshape(-1),
+                 rest.reshape(-1)]
+        dev_info = torch.from_numpy(np.concatenate(parts)).to(device)
         seq_info = dev_info[: 3 * self.S].view(3, self.S)
-        tables = dev_info[3 * self.S:].view(self.S, self.width)
+        end = 3 * self.S + self.tables.size
+        tables = dev_info[3 * self.S: end].view(self.S, self.width)
+        if len(tiles):
+            meta.prefill_tiles = dev_info[end: end + tiles.size].view(-1, 4)
+            meta.prefill_tiles_host = torch.from_numpy(tiles)
+            if rest.size:
+                rows = dev_info[end + tiles.size:].view(3, -1)
+                meta.rest_rows, meta.rest_table, meta.rest_context = rows
         meta.block_tables = tables
         if self.T:
             meta.slot_mapping, meta.row_table, meta.row_context = _native_ops(device).attention_metadata(
@@ -420,6 +467,32 @@ def _attend_torch(q: torch.Tensor, k_cache, v_cache, meta: AttentionMetadata, sc
     out[idx] = od.squeeze(1)
 
 
+def _tiles_ok(q: torch.Tensor, k: torch.Tensor, meta: AttentionMetadata) -> bool:
+    """Batches whose prompt tokens the tiled prefill kernel takes; the row kernel has the rest."""
+    t, hq, d = q.shape
+    hk, bs = k.shape[1], meta.block_size
+    return (meta.prefill_tiles is not None and d in (64, 128) and hq % hk == 0 and hq // hk <= 8
+            and t < 2**24 and hk <= 4096 and len(meta.prefill_tiles_host) < 65536
+            and meta.block_tables.shape[1] * bs < 2**30 and k.shape[0] * hk < 2**31)
+
+
+def _attend_native(ops, q: torch.Tensor, cache, q_mult, meta: AttentionMetadata,
+                   scale: float) -> torch.Tensor:
+    """Every token of the batch over the cache (K, V, K scales, V scales)."""
+    if not _tiles_ok(q, cache[0], meta) or q.shape[0] != meta.row_table.numel():
+        return ops.paged_attention_rows(q, *cache, meta.block_tables, meta.row_table,
+                                        meta.row_context, meta.block_size, scale, q_mult)
+    out = torch.empty_like(q)
+    ops.paged_attention_prefill_(out, q, *cache, meta.block_tables, meta.prefill_tiles,
+                                 meta.prefill_tiles_host, meta.block_size, scale, q_mult)
+    if meta.rest_rows is not None:
+        o = ops.paged_attention_rows(q.index_select(0, meta.rest_rows), *cache, meta.block_tables,
+                                     meta.rest_table, meta.rest_context, meta.block_size, scale,
+                                     q_mult)
+        out.index_copy_(0, meta.rest_rows, o)
+    return out
+
+
 def paged_attention(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -443,16 +516,11 @@ def paged_attention(
         v_cache.write(meta.slot_mapping, v)
     else:
         write_kv(k_cache, v_cache, k, v, meta.slot_mapping)
-    if ops is not None:  # every token is a query row of one native launch
+    if ops is not None:
         q_mult = k_cache._q_mult if smooth is not None else None
-        if quantized:
-            return ops.paged_attention_rows(q.float().contiguous(), k_cache.data, v_cache.data,
-                                            k_cache.scale, v_cache.scale, meta.block_tables,
-                                            meta.row_table, meta.row_context, meta.block_size,
-                                            scale, q_mult)
-        return ops.paged_attention_rows(q.float().contiguous(), k_cache, v_cache, None, None,
-                                        meta.block_tables, meta.row_table, meta.row_context,
-                                        meta.block_size, scale, None)
+        data = (k_cache.data, v_cache.data, k_cache.scale, v_cache.scale) if quantized else (
+            k_cache, v_cache, None, None)
+        return _attend_native(ops, q.float().contiguous(), data, q_mult, meta, scale)
     q_att = q * k_cache._q_mult if smooth is not None else q
     out = torch.empty_like(q)
     _attend_torch(q_att, k_cache, v_cache, meta, scale, out)

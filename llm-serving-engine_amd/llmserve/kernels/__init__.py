@@ -22,7 +22,8 @@ Functions, with the reference's names and signatures where the reference has the
   v_scale, block_tables, context_lens, block_size, scale, partition_size=0, q_mult=None)`` and
   ``paged_attention_decode(q, k_cache, v_cache, block_tables, context_lens, block_size, scale,
   partition_size=0)`` (fp32 cache) (paged_attention.cpp:386-399); ``paged_attention_rows``
-  (every token of a ragged batch as one query row, decode and prefill alike) and
+  (every token of a ragged batch as one query row, decode and prefill alike),
+  ``paged_attention_prefill_`` (prompt tokens in tiles, on the matrix cores) and
   ``attention_metadata`` (slots and query rows of a step, on the device).
 * ``load_quant()``: the load-time quantizers and the int8 KV-cache write.
 * ``load_fused_ops()``: ``rmsnorm``, ``add_rmsnorm_``, ``silu_mul``, ``rope_qk_``
@@ -112,7 +113,8 @@ def load_paged_attention() -> SimpleNamespace | None:
         v1 = None
     return _namespace("paged attention kernels", (
         "paged_attention_decode_int8", "paged_attention_decode_int8_xfrag",
-        "paged_attention_decode", "paged_attention_rows", "attention_metadata"),
+        "paged_attention_decode", "paged_attention_rows", "paged_attention_prefill_",
+        "attention_metadata"),
         paged_attention_decode_v1=v1, set_simd=_set_simd, simd_available=_simd_available)
 
 
