@@ -6,12 +6,12 @@
 // context once per token and runs on the VALU (2 prompts of ~900 tokens after ~1000 cached ones and 24
 // decode rows: 962 us). Here a workgroup takes 64 query tokens and two query heads of one kv head and
 // walks the context in tiles of 64 tokens (fp32 cache: 32) that its four wavefronts share: 87 us for
-// the two prompts, 1000 new tokens over the fp32 cache 776 -> 66.
+// the two prompts, 1000 new tokens over the fp32 cache 776 -> 64.
 //
 // Precision is fp32's: q, the weights and fp32 K / V rows are each split into two fp16 pieces (22
 // bits) after scaling by a power of two (per query row and head, per cache row); int8 codes are exact
 // in fp16, their scales stay in fp32 on the score and on the weight. Products are exact and summed in
-// fp32. Measured against float64: 1.4-3.1e-7 (int8), the row kernel 3.0e-7.
+// fp32. Measured against float64, 1000 new tokens: int8 1.5e-7, fp32 1.6e-7 (the row kernel 3.0e-7, 1.6e-7).
 //
 // Both products are transposed: S^T = K Q^T leaves lane (fr, fc) the scores of query fr for tokens
 // 16 tt + 4 fc + e, which is the B operand layout of O^T = V^T P^T when the k order of that product is
@@ -46,13 +46,17 @@ constexpr int kWaves = 4;
 constexpr int kFrag = 1024;     // bytes of a fragment: 64 lanes x 8 fp16
 constexpr float kLog2e = 1.4426950408889634f;
 // Weights: p = exp2(score - ref), ref the running max of score + log2(v scale) (so that p v_scale
-// stays below 2^kLazy: the reference moves only past that), times v_scale kUp, which brings the fp16
-// pieces near the top of their range. kUp is a factor of the staged v scales rather than of p: p's
-// exponent stays small, and with it the rounding of its argument.
-constexpr float kLazy = 4.f, kUp = 2048.f;
+// stays below 2^kLazy: the reference moves only past that), times v_scale 2^up, which brings the fp16
+// pieces near the top of their range. 2^up is a factor of the staged v scales rather than of p, and a
+// chunk takes it from its first token's v scale (kTop - log2 of it, within kUpMin .. kUpMax), so that
+// the scales it stages are near 2^kTop: p's exponent stays small, and with it the rounding of its
+// argument (with 2^kTop for all the arguments reach 13 and a chunk's reference 20, rounded as such:
+// float64 error over the fp32 cache 2.2e-7 instead of 1.6e-7).
+constexpr float kLazy = 4.f;
+constexpr int kTop = 11, kUpMin = -5, kUpMax = 23;
 // A v scale that is not finite is staged as kHuge, so that a weight of 0 (a token that the query does
 // not see) times it stays 0; a weight that is not 0 still overflows fp16, as the reference follows
-// v scales up to 2^kMaxLv only, and the output is NaN.
+// staged v scales up to 2^(kTop + kMaxLv) only (scales of 2^88 at least), and the output is NaN.
 constexpr float kHuge = 3.402823466e38f, kMaxLv = 100.f;
 
 struct PrefillArgs {
@@ -229,16 +233,38 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
     }
   }
 
+  // ---- staged v scales: times 2^up, from the first token if the tile's first row (so all) sees it --
+  const int64_t* bt = a.bt + static_cast<int64_t>(tab) * a.max_blocks;
+  auto block_of = [&](int t) { return a.bs_shift >= 0 ? t >> a.bs_shift : t / a.bs; };
+  const int64_t blocks = a.num_slots / a.bs, rstride = static_cast<int64_t>(a.Hk) * kRow;
+  int up = kTop;
+  {
+    const int64_t id0 = k0 < sees ? bt[block_of(k0)] : static_cast<int64_t>(-1);
+    if (id0 >= 0 && id0 < blocks) {
+      const int64_t slot0 = id0 * a.bs + (k0 - block_of(k0) * a.bs);
+      float v0 = 0.f;
+      if constexpr (kF32) {
+        const float* vp = reinterpret_cast<const float*>(static_cast<const char*>(a.vc) + slot0 * rstride + kvh * kRow);
+#pragma unroll
+        for (int i = 0; i < D / kWave; ++i) v0 = fmaxf(v0, fabsf(vp[i * kWave + lane]));
+        v0 = lsh::wave_max_from<1>(v0) * 0x1p-15f;
+      } else {
+        v0 = a.vs[slot0 * a.Hk + kvh];
+      }
+      if (v0 > 0.f && v0 < __builtin_inff())
+        up = min(max(kTop - __builtin_amdgcn_frexp_expf(v0), kUpMin), kUpMax);
+    }
+    up = __builtin_amdgcn_readfirstlane(up);
+  }
+  const float v_up = __builtin_bit_cast(float, static_cast<uint32_t>(up + 127) << 23);
+
   // ---- staging: wavefront w brings tokens TW w .. + TW of a context tile ------------------------
   // block id of the token this lane looks after (lane % TW of the wavefront's), read a tile ahead
-  const int64_t* bt = a.bt + static_cast<int64_t>(tab) * a.max_blocks;
   auto token_of = [&](int it) { return k0 + it * KT + TW * wave + lane % TW; };
-  auto block_of = [&](int t) { return a.bs_shift >= 0 ? t >> a.bs_shift : t / a.bs; };
   auto fetch_id = [&](int it) {
     const int t = token_of(it);
     return t < k1 ? bt[block_of(t)] : static_cast<int64_t>(-1);
   };
-  const int64_t blocks = a.num_slots / a.bs, rstride = static_cast<int64_t>(a.Hk) * kRow;
   auto slot_of = [&](int it, int64_t id) {  // cache slot, -1: no such token
     const int t = token_of(it);
     return id < 0 || id >= blocks ? -1 : static_cast<int>(id) * a.bs + (t - block_of(t) * a.bs);
@@ -316,7 +342,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
         *reinterpret_cast<u32x2*>(v_at(conv, 0, d + 3, vg)) = u32x2{bytes_to_h2<0x04030402u>(q01), bytes_to_h2<0x04030402u>(q23)};
       }
       if (lane < TW) sk[TW * wave + lane] = scale;
-      if (lane >= TW && lane < 2 * TW) sv[TW * wave + lane - TW] = fminf(scale * kUp, kHuge);
+      if (lane >= TW && lane < 2 * TW) sv[TW * wave + lane - TW] = fminf(scale * v_up, kHuge);
     } else {
       // a row's exponent, from the largest magnitude as an integer (NaN and infinity above all)
       auto row_scale = [&](uint32_t top, int lanes, float& up) {
@@ -361,7 +387,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
       for (int t = 0; t < 4; ++t) {
         r[t] = *reinterpret_cast<const u32x4*>(raw[wave][1] + (vl0 + t) * kRow + vd0 * 4);
         const float down = row_scale(mag(r[t]), kVLanes, up[t]);
-        if (v_on && vd0 == 0) sv[4 * vg + t] = ok >> (vl0 + t) & 1 ? fminf(down * kUp, kHuge) : 0.f;
+        if (v_on && vd0 == 0) sv[4 * vg + t] = ok >> (vl0 + t) & 1 ? fminf(down * v_up, kHuge) : 0.f;
       }
       if (v_on) {
 #pragma unroll
@@ -409,8 +435,8 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
     for (int tt = 0; tt < TT; ++tt) {
       // Two sums per score, added at the end: the first half of the hi products in one, the rest, with
       // the small products of lo pieces, in the other. One chain would round at the score's size three
-      // times as often: measured error against float64 2.1e-7 with one, 1.7e-7 with two (int8, 1000
-      // tokens); more than two change nothing.
+      // times as often; more than two change nothing. lo lo products are small but not nothing:
+      // float64 error over the fp32 cache 1.61e-7 without them, 1.57e-7 with.
       f32x4 part[kHeads][2] = {};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
@@ -425,6 +451,8 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
         if constexpr (PL == 2) {
 #pragma unroll
           for (int c2 = 0; c2 < kHeads; ++c2) part[c2][1] = mfma(kf[1], qf[c2][ks][0], part[c2][1]);
+#pragma unroll
+          for (int c2 = 0; c2 < kHeads; ++c2) part[c2][1] = mfma(kf[1], qf[c2][ks][1], part[c2][1]);
         }
 #pragma unroll
         for (int c2 = 0; c2 < kHeads; ++c2) part[c2][half] = mfma(kf[0], qf[c2][ks][0], part[c2][half]);
@@ -432,7 +460,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
 #pragma unroll
       for (int c2 = 0; c2 < kHeads; ++c2) s[c2][tt] = part[c2][0] + part[c2][1];
     }
-    read_ahead<TT * KS, PL, kHeads * (PL + 1)>();
+    read_ahead<TT * KS, PL, kHeads * (PL == 2 ? 4 : 2)>();
     __builtin_amdgcn_s_setprio(0);
     // scores (times qs: log2 units); lane (fr, fc) holds tokens 16 tt + 4 fc + e of its query
     float vtop = 0.f;  // the largest v scale
@@ -468,7 +496,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
         }
       }
     }
-    const float lv = fminf(fmaxf(__builtin_amdgcn_logf(max_over_fc(vtop) * (1.f / kUp)), -kMaxLv), kMaxLv);
+    const float lv = fminf(fmaxf(__builtin_amdgcn_logf(max_over_fc(vtop)) - kTop, -kMaxLv), kMaxLv);
     float top[kHeads];
     bool raise = false;
 #pragma unroll
@@ -506,13 +534,14 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
 #pragma unroll
       for (int c = 0; c < kHeads; ++c) {
         u32x4 hi, lo;
+        float eight = 0.f;  // added up apart: an eighth of the roundings at the sum's size
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           float w[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[c][2 * vs + h][e], qs[c], -ref[c]));
-            sum[c] += p;
+            eight += p;
             w[e] = p * vsc[h][e];
           }
           uint32_t h0, l0, h1, l1;
@@ -523,6 +552,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
           lo[2 * h] = l0;
           lo[2 * h + 1] = l1;
         }
+        sum[c] += eight;
         ph[c] = __builtin_bit_cast(f16x8, hi);
         pl[c] = __builtin_bit_cast(f16x8, lo);
       }
@@ -559,7 +589,7 @@ if constexpr (PL == 1) {
     const float l = sum_over_fc(sum[c]);
     if (16 * wave + fr >= rows || g0 + c >= a.G) continue;
     if (whole) {
-      const float inv = 1.f / (l * kUp);
+      const float inv = 1.f / (l * v_up);
       float* o = a.out + (static_cast<int64_t>(row0 + tok) * a.Hq + head[c]) * D + 4 * fc;
 #pragma unroll
       for (int d = 0; d < DT; ++d)
@@ -568,9 +598,9 @@ if constexpr (PL == 1) {
       const int64_t at = (((static_cast<int64_t>(tile) * a.Hk * a.pairs + hp) * a.splits + chunk) * kHeads + c) * kQT + tok;
       float* o = a.part_acc + at * D + 4 * fc;
 #pragma unroll
-      for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4*>(o + 16 * d) = acc[c][d];
+      for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4*>(o + 16 * d) = acc[c][d] * (1.f / v_up);
       if (fc == 0) {
-        a.part_rl[2 * at] = ref[c];
+        a.part_rl[2 * at] = ref[c];  // as the weights used it: any sum with it would round
         a.part_rl[2 * at + 1] = l;
       }
     }
@@ -621,7 +651,7 @@ __global__ __launch_bounds__(kWaves* kWave) void prefill_merge_kernel(PrefillArg
       for (int e = 0; e < 4; ++e) o[e] += w * (on ? v[j][e] : 0.f);
     }
   }
-  const float inv = 1.f / (L * kUp);
+  const float inv = 1.f / L;
   *reinterpret_cast<f32x4*>(a.out + (a.tiles[4 * tile] + tok) * a.Hq * D + static_cast<int64_t>(h) * D + 4 * part) =
       o * inv;
 }
