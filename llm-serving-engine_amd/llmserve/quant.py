@@ -252,11 +252,14 @@ class Int4Linear(nn.Module):
 
     def _tile_ok(self, x: torch.Tensor) -> bool:
         """Inputs the tiled GEMM (int4_linear_tile) takes; the others keep the torch ops, which
-        differentiate and promote types."""
+        differentiate (also through the scales), promote types and follow autocast."""
         rows, (n, k) = x.shape[0], (self.out_features, self.in_features)
         return (k % 128 == 0 and self.group_size % 64 == 0 and x.dtype == torch.float32
                 and rows < 2**24 and n < 2**22 and k < 2**20 and rows * k < 2**36
-                and not (x.requires_grad and torch.is_grad_enabled())
+                and not (torch.is_grad_enabled() and any(
+                    t is not None and t.requires_grad
+                    for t in (x, self.g_scale, self.g_zero, self.inv_act_scale)))
+                and not torch.is_autocast_enabled(x.device.type)
                 and torch.autograd.forward_ad._current_level < 0)
 
     def _path(self, rows: int, native, x: torch.Tensor | None = None) -> str:

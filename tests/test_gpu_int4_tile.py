@@ -97,3 +97,19 @@ def test_module_dispatch(gpu, group, rows, path):
     assert not Int4Linear(torch.nn.Linear(192, 8, device="cuda"), 64)._tile_ok(x[:, :192])
     assert torch.ops.llmserve_hip.int4_linear_tile(
         *(t.to("meta") for t in (x, m.nibbles, m.g_scale, m.g_zero)), group).shape == y.shape
+
+
+@pytest.mark.parametrize("name", ["x", "g_scale", "g_zero"])
+def test_gradients_and_autocast_keep_the_torch_ops(gpu, name):
+    from llmserve.quant import Int4Linear
+
+    m = Int4Linear(torch.nn.Linear(256, 40, bias=False, device="cuda"), 64)
+    x = torch.randn(33, 256, device="cuda")
+    assert m._tile_ok(x)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not m._tile_ok(x) and m(x).dtype == torch.bfloat16
+    t = (x if name == "x" else getattr(m, name)).requires_grad_()
+    m(x).sum().backward()
+    assert t.grad is not None and t.grad.abs().sum() > 0
+    with torch.no_grad():
+        assert m._tile_ok(x)
