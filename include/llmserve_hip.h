@@ -226,7 +226,8 @@ int llmserve_int4_linear_gemm_xfrag_split(const void* xfrag, const void* packed,
  * 64; x, q and the workspace 16-byte aligned; the workspace holds
  * llmserve_int8_linear_prefill_workspace_bytes(M, N, K) bytes: the bf16 copy of x and, when
  * the output has fewer 256 x 256 tiles than the device has CUs, the fp32 partial sums of the
- * K splits (their count depends on the current device).
+ * K splits (their count depends on the current device); for small products (M N K up to 12 * 2^30,
+ * K a multiple of 128) bf16(x) as fp16 fragments of rows scaled by a power of two.
  */
 int64_t llmserve_int8_linear_prefill_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int llmserve_int8_linear_prefill(const float* x, const int8_t* qweight, const float* scale,

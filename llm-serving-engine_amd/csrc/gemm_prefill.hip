@@ -5,6 +5,8 @@
 // (reference quant.py:71-72, dequantize :78-79: x @ (q * scale[:, None]).T) with the
 // per-channel scale moved to the epilogue.
 //
+// Calls with little work for 256 x 256 tiles go to gemm_tile.hip (use_tiles below).
+//
 // Tiling: a 512-thread workgroup owns a 256 x 256 output tile (or, split-K, one K range of
 // it); its eight wavefronts (two per SIMD, so one waits for LDS or a barrier while the other
 // issues MFMAs) own 128 x 64 parts, each a grid of 8 x 4 v_mfma_f32_16x16x32_bf16 tiles (128
@@ -25,7 +27,7 @@
 // Units map to blocks XCD-aware: block b runs on XCD b % 8, and each XCD gets whole columns
 // of units (a tile column and its splits), so a weight panel is read from HBM into one XCD's
 // L2 and reused there by every row tile of the column.
-#include "common.h"
+#include "gemm_tile.h"
 
 namespace {
 
@@ -271,10 +273,22 @@ int prefill_splits(int64_t M, int64_t N, int64_t K) {
   return s;
 }
 
+// Products that go to the small tiles of gemm_tile.hip (the same products of bf16(x), exact in fp16).
+// A 256 x 256 tile is mostly padding at few rows, and up to about 12 G products the tiles and K splits
+// here leave CUs idle or pay for the partial sums (us, here / small tiles, K x N):
+//   32 rows: 1024 x 6144 20.4 / 9.5, 2048 x 1024 24.6 / 12.2; 256: 1024 x 4096 37.8 / 13.1, 2048 x 16384 53 / 46;
+//   1024: 2048 x 6144 62 / 45; 2048: 1024 x 6144 43.8 / 42.0 (the line);
+// above it the small tiles read x and the weight too often:
+//   777: 8192 x 2048 81.6 / 82.0, 2048 x 16384 73 / 85; 2048: 2048 x 6144 66 / 69, 8192 x 2048 106 / 164.
+bool use_tiles(int64_t M, int64_t N, int64_t K) {
+  return K % 128 == 0 && M <= (12LL << 30) / (N * K);
+}
+
 }  // namespace
 
 extern "C" int64_t llmserve_int8_linear_prefill_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (use_tiles(M, N, K)) return lsh::int8_tile_workspace_bytes(M, N, K);
   const int64_t xb = (M * K * 2 + 255) / 256 * 256;  // bf16 copy of x
   const int s = prefill_splits(M, N, K);
   return xb + (s > 1 ? s * M * N * static_cast<int64_t>(sizeof(float)) : 0);
@@ -299,6 +313,10 @@ extern "C" int llmserve_int8_linear_prefill(const float* x, const int8_t* qweigh
             "int8_linear_prefill: 16-byte aligned workspace of %lld bytes needed, %lld given",
             (long long)need, (long long)workspace_bytes);
   hipStream_t st = lsh::as_stream(stream);
+  if (use_tiles(M, N, K)) {
+    lsh::int8_tile_launch(x, qweight, scale, y, M, N, K, workspace, st);
+    return lsh::launch_status("int8_linear_prefill");
+  }
   __bf16* xb = static_cast<__bf16*>(workspace);
   const int64_t n4 = M * K / 4;
   const int64_t cgrid = (n4 + 255) / 256 < 4096 ? (n4 + 255) / 256 : 4096;

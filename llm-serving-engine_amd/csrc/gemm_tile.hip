@@ -2,11 +2,13 @@
 //   int4:  y[m, n] = sum_g s[n, g] sum_{k in g} x'[m, k] q[n, k] + (z - 8 s)[n, g] sum_{k in g} x'[m, k]
 //          with x' = x * inv_act_scale (Int4Linear.forward's large-M branch, reference
 //          quant.py:141-142, in the group decomposition of int8_gemv.cpp:48-52).
+//   int8:  y[m, n] = scale[n] sum_k bf16(x[m, k]) q[n, k], llmserve_int8_linear_prefill's product
+//          (gemm_prefill.hip says for which sizes it comes here).
 // Operands: q is exact in fp16. Each row of x' is scaled by the power of two that brings its
 // largest value to [2^14, 2^15) and split into two fp16 pieces, hi = fp16(x'), lo = fp16(x' - hi):
-// 22 significant bits, down to 2^-38 of the row's largest value. Products are exact in fp32 and
-// summed there. Measured against float64: 2.7-3.3e-7 relative (the two bfloat16 pieces of
-// int4_gemm_mfma 5.3e-6, dequantize + fp32 GEMM 8e-7).
+// 22 significant bits, down to 2^-38 of the row's largest value (int8: bf16(x) is one piece, exact
+// down to 2^-31 of it). Products are exact in fp32 and summed there. Measured against float64: 2.7-3.3e-7
+// relative (the two bfloat16 pieces of int4_gemm_mfma 5.3e-6, dequantize + fp32 GEMM 8e-7).
 //
 // Two launches. The split pass (one wavefront per row) writes the pieces as MFMA fragments, the
 // sums of x' over each unit of constant group scale, and the constants z - 8 s; for a weight in
@@ -26,7 +28,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "common.h"
+#include "gemm_tile.h"
 
 namespace {
 
@@ -88,6 +90,7 @@ __device__ __forceinline__ uint32_t as_u(f16x2 h) { return __builtin_bit_cast(ui
 __device__ __forceinline__ int exponent_to_15(float top) {  // 2^result brings top to [2^14, 2^15)
   int ex = 0;
   if (top > 0.f && top < __builtin_inff()) ex = 15 - __builtin_amdgcn_frexp_expf(top);
+  if (top == __builtin_inff()) ex = -113;  // the largest finite value then stays finite in fp16
   return ex < -126 ? -126 : (ex > 126 ? 126 : ex);
 }
 
@@ -266,7 +269,7 @@ __global__ __launch_bounds__(kSplitRows* kWave) void split_rows_kernel(
   const int total = nblk * (kBlk / 8);  // chunks of the padded row
   auto put = [&](int c, float (&v)[8]) {  // every lane calls it (a unit's sum crosses lanes)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] *= up;
+    for (int e = 0; e < 8; ++e) v[e] = (O == kInt8 ? static_cast<float>(static_cast<__bf16>(v[e])) : v[e]) * up;
     // chunk cc of block b -> (q, fc)
     const int b = c / 16, cc = c % 16;
     const int q = O == kInt4G128 ? cc % 4 : 2 * (cc / 8) + cc % 2;
@@ -690,6 +693,23 @@ void run_tile(const float* x, const float* inv, const WeightIn& in, const TileAr
 }
 
 }  // namespace
+
+int64_t lsh::int8_tile_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  return lay_out<kInt8>(nullptr, M, N, K, 0, false, nullptr);
+}
+
+void lsh::int8_tile_launch(const float* x, const int8_t* qweight, const float* scale, float* y, int64_t M, int64_t N,
+                           int64_t K, void* workspace, hipStream_t st) {
+  TileArgs a{};
+  lay_out<kInt8>(static_cast<char*>(workspace), M, N, K, 0, false, &a.a);
+  a.w = reinterpret_cast<const uint8_t*>(qweight);
+  a.s = scale;
+  a.y = y;
+  a.M = static_cast<int>(M);
+  a.N = static_cast<int>(N);
+  a.K = static_cast<int>(K);
+  run_tile<kInt8>(x, nullptr, WeightIn{}, a, st);
+}
 
 extern "C" int64_t llmserve_int4_linear_tile_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size) {
   if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || K % kBlk || group_size % 64 || K % group_size) return 0;

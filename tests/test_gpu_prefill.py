@@ -100,3 +100,33 @@ def test_rejects_bad_k(gpu):
     s = torch.ones(8, device="cuda")
     with pytest.raises(RuntimeError, match="multiple of 64"):
         cu.int8_linear_prefill(x, q, s)
+
+
+# Both sides of the line between the small tiles and the 256-wide ones, at the small tiles' edges (16 x 64,
+# 32 x 128, 64 x 256 with 4, 2 and 1 K parts), odd row and channel counts and K block counts that
+# pad; K off the 128 grid stays with the 256-wide tiles.
+@pytest.mark.parametrize("M,N,K", [(1, 1, 128), (17, 63, 256), (16, 65, 384), (33, 1000, 640), (129, 257, 1152),
+                                   (777, 1025, 512), (1290, 4161, 384), (2048, 6144, 1024),
+                                   (2049, 6144, 1024), (33, 1000, 704)])
+def test_small_tiles(gpu, M, N, K):
+    x, q, s = make(M + N + K, M, N, K)
+    x[:, 3] *= 1000  # a channel far above the others
+    y = cu.int8_linear_prefill(cu.dev(x), cu.dev(q), cu.dev(s))
+    check(y, x, q, s, np.random.default_rng(M).permutation(M)[:200])
+
+
+def test_small_tiles_rows_are_independent(gpu):
+    """Rows of 1e-30 .. 1e30, a zero row, an infinity (beside the largest finite values) and a NaN: each
+    row as float32 arithmetic on bf16(x) has it."""
+    x, q, s = make(3, 40, 96, 256)
+    x[:8] *= np.logspace(-30, 30, 8).astype(F32)[:, None]
+    x[8] = 0
+    x[9] = 1e38
+    x[9, 200], x[10, 3] = np.inf, np.nan
+    y = cu.int8_linear_prefill(cu.dev(x), cu.dev(q), cu.dev(s)).cpu().numpy()
+    want = np.where(q[:, 200] == 0, np.nan, np.sign(q[:, 200]) * np.inf)
+    np.testing.assert_array_equal(y[9], want.astype(F32))
+    assert np.isnan(y[10]).all() and not y[8].any()
+    for r in (r for r in range(40) if r not in (8, 9, 10)):
+        exact = mr.int8_linear_prefill_f64(x[r:r + 1], q, s)
+        assert rel_l2(y[r:r + 1], exact) <= TIGHT_L2, r
