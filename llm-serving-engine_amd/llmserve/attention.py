@@ -468,10 +468,10 @@ def _attend_torch(q: torch.Tensor, k_cache, v_cache, meta: AttentionMetadata, sc
 
 
 def _tiles_ok(q: torch.Tensor, k: torch.Tensor, meta: AttentionMetadata) -> bool:
-    """Batches whose prompt tokens the tiled prefill kernel takes; the row kernel has the rest."""
+    """Whether the tiled prefill kernel takes the batch's tiles; the row kernel has the rest."""
     t, hq, d = q.shape
     hk, bs = k.shape[1], meta.block_size
-    return (meta.prefill_tiles is not None and d in (64, 128) and hq % hk == 0 and hq // hk <= 8
+    return (d in (64, 128) and hq % hk == 0 and hq // hk <= 8
             and t < 2**24 and hk <= 4096 and len(meta.prefill_tiles_host) < 65536
             and meta.block_tables.shape[1] * bs < 2**30 and k.shape[0] * hk < 2**31)
 
@@ -479,7 +479,8 @@ def _tiles_ok(q: torch.Tensor, k: torch.Tensor, meta: AttentionMetadata) -> bool
 def _attend_native(ops, q: torch.Tensor, cache, q_mult, meta: AttentionMetadata,
                    scale: float) -> torch.Tensor:
     """Every token of the batch over the cache (K, V, K scales, V scales)."""
-    if not _tiles_ok(q, cache[0], meta) or q.shape[0] != meta.row_table.numel():
+    if (meta.prefill_tiles is None or not _tiles_ok(q, cache[0], meta)
+            or q.shape[0] != meta.row_table.numel()):
         return ops.paged_attention_rows(q, *cache, meta.block_tables, meta.row_table,
                                         meta.row_context, meta.block_size, scale, q_mult)
     out = torch.empty_like(q)
