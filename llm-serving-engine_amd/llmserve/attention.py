@@ -171,17 +171,21 @@ class _BatchPlan:
         context) for the native backend."""
         tiled = (self.q >= TILE_ROWS) & (self.ctx >= self.q)
         seqs = np.flatnonzero(tiled)
-        gain = ROW_US * float((self.q[seqs] * self.ctx[seqs]).sum()) - TILE_US
-        gain -= CTX_US * float(self.ctx[seqs].max(initial=0)) + (REST_US if seqs.size < self.S else 0)
-        if not seqs.size or gain <= 0:
-            return np.zeros((0, 4), np.int64), np.zeros((3, 0), np.int64)
-        tiles = []
-        for s in seqs.tolist():
-            at = np.arange(0, self.q[s], QUERY_TILE)
-            tiles.append(np.stack([self.q_start[s] + at, np.minimum(QUERY_TILE, self.q[s] - at),
-                                   self.ctx[s] - self.q[s] + at + 1, np.full_like(at, s)], axis=1))
-        tiles = np.concatenate(tiles)
-        tiles = np.ascontiguousarray(tiles[np.argsort(-(tiles[:, 1] + tiles[:, 2]), kind="stable")])
+        none = np.zeros((3, 0), np.int64)
+        if not seqs.size:
+            return np.zeros((0, 4), np.int64), none
+        q, ctx = self.q[seqs], self.ctx[seqs]
+        gain = ROW_US * float((q * ctx).sum()) - TILE_US - CTX_US * float(ctx.max())
+        if gain <= (REST_US if seqs.size < self.S else 0):
+            return np.zeros((0, 4), np.int64), none
+        counts = -(-q // QUERY_TILE)
+        of = np.repeat(np.arange(seqs.size), counts)  # the tiles' sequences, as indices into seqs
+        at = QUERY_TILE * (np.arange(of.size) - (np.cumsum(counts) - counts)[of])
+        n, first = np.minimum(QUERY_TILE, q[of] - at), (ctx - q)[of] + at + 1
+        order = np.argsort(-(n + first), kind="stable")
+        tiles = np.stack([self.q_start[seqs][of] + at, n, first, seqs[of]], axis=1)[order]
+        if seqs.size == self.S:
+            return tiles, none
         seq, pos = self.token_positions()
         rest = np.flatnonzero(~tiled[seq])
         return tiles, np.stack([rest, seq[rest], pos[rest] + 1])
