@@ -599,8 +599,9 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_tile_kernel(TileArgs a)
     }
   }
 
-  // lane holds rows 4 fc + e, column fr of each 16 x 16 tile; stores past the last row or
-  // channel fall outside the buffer and are dropped
+  // lane holds rows 4 fc + e, column fr of each 16 x 16 tile; a store past the last row or channel
+  // gets a vector offset outside the buffer and is dropped (the scalar offset takes no part in the
+  // bounds check, so the row must not go there)
   const int m0 = tm * TM * 16;
   const auto ry = rsrc(a.y + static_cast<int64_t>(m0) * a.N, static_cast<int64_t>(a.M - m0) * a.N * 4);
   f32x4 rm[TM];  // before the stores: a load behind them would wait for them
@@ -612,15 +613,17 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_tile_kernel(TileArgs a)
 #pragma unroll
   for (int t = 0; t < TM; ++t)
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+    for (int e = 0; e < 4; ++e) {
+      const int row = 16 * t + 4 * fc + e;
+      const uint32_t row_ofs = static_cast<uint32_t>(row) * static_cast<uint32_t>(a.N) * 4;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int n = n0 + 16 * u + fr;
-        const uint32_t ofs = n < a.N ? static_cast<uint32_t>((4 * fc * a.N + n) * 4) : 0x80000000u;
+        const uint32_t ofs = n < a.N && m0 + row < a.M ? row_ofs + static_cast<uint32_t>(n) * 4 : 0x80000000u;
         const float v = O == kInt8 ? acc[t][u][e] * cs[u] : acc[t][u][e];
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v * rm[t][e]), ry, ofs,
-                                              (16 * t + e) * a.N * 4, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v * rm[t][e]), ry, ofs, 0, 0);
       }
+    }
 }
 
 // The workspace laid out at p; returns the bytes it takes.

@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 import torch
 
+import capi_util as cu
 from llmserve.kernels import load_int8_gemv
 from oracle import math_ref as mr
 from oracle import quant as oq
@@ -113,3 +114,35 @@ def test_gradients_and_autocast_keep_the_torch_ops(gpu, name):
     assert t.grad is not None and t.grad.abs().sum() > 0
     with torch.no_grad():
         assert m._tile_ok(x)
+
+
+# each tile (16 x 64, 32 x 128, 64 x 256) with its last row tile partly past M, down to one row in it
+@pytest.mark.parametrize("M,N,K", [(1, 60, 128), (17, 64, 256), (33, 70, 128), (65, 136, 384), (33, 12200, 128),
+                                   (65, 12300, 128), (65, 41000, 128), (1281, 4100, 128)])
+@pytest.mark.parametrize("weights", ["int4", "int8"])
+def test_nothing_is_written_behind_y(gpu, M, N, K, weights):
+    """The bytes behind y and behind the workspace stay as they were."""
+    pad = 64 * N  # floats: more than the rows a tile can have past M
+    rng = np.random.default_rng(M + N)
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(F32)).cuda()
+    w = torch.from_numpy((rng.standard_normal((N, K)) * 0.02).astype(F32)).cuda()
+    y = torch.full((M * N + pad,), -7.5, device="cuda")
+    lib = cu.capi()
+    if weights == "int8":
+        q, s = cu.int8_quantize(w)
+        need = lib.llmserve_int8_linear_prefill_workspace_bytes(M, N, K)
+    else:
+        q, gs, gz, _ = cu.int4_quantize(w, 64)
+        need = lib.llmserve_int4_linear_tile_workspace_bytes(M, N, K, 64)
+    ws = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    if weights == "int8":
+        cu.check(lib.llmserve_int8_linear_prefill(cu._p(x), cu._p(q), cu._p(s), cu._p(y), M, N, K, cu._p(ws), need,
+                                                  cu._stream()))
+        ref = x.bfloat16().double() @ (q.double() * s.double()[:, None]).t()
+    else:
+        cu.check(lib.llmserve_int4_linear_tile(cu._p(x), None, cu._p(q), cu._p(gs), cu._p(gz), None, cu._p(y), M, N,
+                                               K, 64, cu._p(ws), need, cu._stream()))
+        ref = mr.int4_linear_f64(*(t.cpu().numpy() for t in (x, q, gs, gz)), 64)
+        ref = torch.from_numpy(ref).cuda()
+    assert (y[M * N:] == -7.5).all() and (ws[need:] == 0x5A).all()
+    assert (y[: M * N].view(M, N) - ref).norm() <= 2e-6 * ref.norm()
