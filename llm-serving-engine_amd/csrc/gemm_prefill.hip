@@ -115,23 +115,26 @@ __global__ __launch_bounds__(kThreads, 1) void int8_gemm_bf16(GemmArgs a) {
   const int wm = wave / 4, wn = wave % 4;  // 128 x 16 NJ part of the tile
   const int K = a.K;
 
-  // Global loads: a lane-constant byte offset, the stage's k (and the row block i) in the
-  // scalar offset. A: rows t / 8 + 64 i, chunk t % 8; B: rows t / 4 + 128 i, 16 bytes t % 4.
+  // Global loads: a lane-constant byte offset per row block, the stage's k in the scalar offset.
+  // A: rows t / 8 + 64 i, chunk t % 8; B: rows t / 4 + 128 i, 16 bytes t % 4. Rows past the
+  // matrix read its last row (their results are not stored): the scalar offset takes no part in
+  // the buffers' bounds check, which would so miss reads past the end.
   const auto ra = rsrc(a.xb, static_cast<int64_t>(a.M) * K * 2);
   const auto rb = rsrc(a.q, static_cast<int64_t>(a.N) * K);
-  const int ga_off = ((m0 + t / 8) * K + 8 * (t % 8)) * 2;
-  const int gb_off = (n0 + t / 4) * K + 16 * (t % 4);
+  int ga_off[4], gb_off[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ga_off[i] = (min(m0 + t / 8 + 64 * i, a.M - 1) * K + 8 * (t % 8)) * 2;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) gb_off[i] = min(n0 + t / 4 + 128 * i, a.N - 1) * K + 16 * (t % 4);
   auto load_a = [&](u32x4 (&ga)[4], int k0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      ga[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                            ra, ga_off, (k0 + i * 64 * K) * 2, 0));
+      ga[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, ga_off[i], k0 * 2, 0));
   };
   auto load_b = [&](u32x4 (&gb)[2], int k0) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      gb[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                            rb, gb_off, k0 + i * 128 * K, 0));
+      gb[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, gb_off[i], k0, 0));
   };
   // LDS stores: the swizzle of rows t / 8 + 64 i (A) and t / 4 + 128 i (B) depends on t only.
   const int sa_off = (t / 8) * 128 + swz(t / 8, t % 8) * 16;

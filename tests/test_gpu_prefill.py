@@ -50,11 +50,24 @@ def make(seed, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 64), (37, 100, 64), (256, 256, 128), (300, 520, 192),
                                    (513, 257, 320), (64, 2048, 1024), (200, 300, 4096),
-                                   (2048, 6000, 128)])  # 192-wide tiles, a 48-column last one
+                                   (2048, 6000, 128)])
 def test_shapes(gpu, M, N, K):
     x, q, s = make(M * 7 + N, M, N, K)
     y = cu.int8_linear_prefill(cu.dev(x), cu.dev(q), cu.dev(s))
     check(y, x, q, s)
+
+
+# The 256-row tiles with their last row and column tiles partly past M and N, above the line to the
+# small tiles: four K splits, 192-wide tiles (a 48-column last one), and K off the 128 grid.
+@pytest.mark.parametrize("M,N,K,splits", [(777, 2040, 8192, 4), (2040, 6000, 2048, 1), (33, 1000, 704, 1)])
+def test_partial_large_tiles(gpu, M, N, K, splits):
+    x, q, s = make(M + N, M, N, K)
+    copy = (M * K * 2 + 255) // 256 * 256
+    partials = splits * M * N * 4 if splits > 1 else 0
+    assert cu.capi().llmserve_int8_linear_prefill_workspace_bytes(M, N, K) == copy + partials
+    y = cu.int8_linear_prefill(cu.dev(x), cu.dev(q), cu.dev(s))
+    rows = np.concatenate([np.arange(min(M, 40)), np.arange(M)[-40:]])
+    check(y, x, q, s, rows)
 
 
 @pytest.mark.parametrize("N,K", [(6144, 2048), (16384, 2048), (2048, 8192)])
