@@ -295,8 +295,10 @@ class Int4Linear(nn.Module):
                                                self.out_features, self.group_size,
                                                self.inv_act_scale)
         elif path == "tile":
+            # The call packs the weight itself, from the buffers as they are now: a write to them
+            # that no version counter sees (through .data, by a kernel) counts too.
             y = native.int4_linear_tile(x2.contiguous(), self.nibbles, self.g_scale, self.g_zero,
-                                        self.group_size, self.inv_act_scale, self.gemm_packed)
+                                        self.group_size, self.inv_act_scale)
         else:
             fn = native.int4_linear if path == "gemv" else native.int4_linear_gemm
             y = fn(x2.contiguous(), self.nibbles, self.g_scale, self.g_zero, self.group_size,

@@ -146,3 +146,32 @@ def test_nothing_is_written_behind_y(gpu, M, N, K, weights):
         ref = torch.from_numpy(ref).cuda()
     assert (y[M * N:] == -7.5).all() and (ws[need:] == 0x5A).all()
     assert (y[: M * N].view(M, N) - ref).norm() <= 2e-6 * ref.norm()
+
+
+def follows(m, x):
+    """The module's output is the product of the buffers it holds now."""
+    with torch.no_grad():
+        y, ref = m(x), x.double() @ m.dequantize().double().t()
+    return (y - ref).norm() <= 1e-5 * ref.norm()
+
+
+@pytest.mark.parametrize("group,rows", [(128, 300), (64, 300), (64, 40)])
+def test_large_batches_follow_the_buffers(gpu, group, rows):
+    """After a state dict, an in-place change, one through .data (that no version counter sees), a new
+    buffer and under functional_call."""
+    from llmserve.quant import Int4Linear
+
+    a, b = (Int4Linear(torch.nn.Linear(256, 208, bias=False, device="cuda"), group) for _ in range(2))
+    x = torch.randn(rows, 256, device="cuda")
+    old = a(x)
+    with torch.no_grad():
+        swapped = torch.func.functional_call(a, dict(b.state_dict()), (x,))
+        assert torch.equal(swapped, b(x)) and torch.equal(a(x), old)
+    a.load_state_dict(b.state_dict())
+    assert follows(a, x) and not torch.equal(a(x), old)
+    a.g_scale.mul_(3)
+    assert follows(a, x)
+    a.g_zero.data.add_(0.5)
+    assert follows(a, x)
+    a.nibbles = torch.flip(a.nibbles, (0,)).contiguous()
+    assert follows(a, x)
