@@ -17,6 +17,7 @@ Kernel switches (class attributes, as in the reference, quant.py:35-37 and :123-
 from __future__ import annotations
 
 import itertools
+import weakref
 from collections import defaultdict
 
 import torch
@@ -208,29 +209,31 @@ class Int4Linear(nn.Module):
             raise ValueError(f"in_features {self.in_features} not divisible by group {group_size}")
         self.group_size = group_size
         dev = _target(linear, device)
-        w = linear.weight.detach().to(device=dev, dtype=torch.float32).contiguous()
-        s = None if act_scale is None else act_scale.detach().to(dev, torch.float32).contiguous()
-        ops = _native("quant", dev)
-        if ops is not None:
-            nib, g_scale, g_zero, inv = ops.int4_quantize(w, group_size, s)
-        else:
-            q, g_scale, g_zero = _int4_groups_torch(w * s[None, :] if s is not None else w,
-                                                    group_size)
-            nib, inv = _pack_nibbles(q), (1.0 / s if s is not None else None)
-        if s is not None:
-            self.register_buffer("inv_act_scale", inv.contiguous())
-        else:
-            self.inv_act_scale = None
-        self.register_buffer("nibbles", nib)  # [out, in / 2]
-        self.register_buffer("g_scale", g_scale.contiguous())  # [out, groups]
-        self.register_buffer("g_zero", g_zero.contiguous())
-        # The weight rearranged for the decode-batch matrix-core kernel (not saved: it is a
-        # function of the three buffers above).
-        packed = None
-        gemv = _native("gemv", dev)
-        if gemv is not None and self.in_features % 128 == 0 and group_size % 128 == 0:
-            packed = gemv.int4_gemm_pack(nib, g_scale, g_zero, group_size)
-        self.register_buffer("gemm_packed", packed, persistent=False)
+        with torch.inference_mode(False):  # buffers with version counters (see _packed_current)
+            w = linear.weight.detach().to(device=dev, dtype=torch.float32).contiguous()
+            s = None if act_scale is None else act_scale.detach().to(dev, torch.float32).contiguous()
+            ops = _native("quant", dev)
+            if ops is not None:
+                nib, g_scale, g_zero, inv = ops.int4_quantize(w, group_size, s)
+            else:
+                q, g_scale, g_zero = _int4_groups_torch(w * s[None, :] if s is not None else w,
+                                                        group_size)
+                nib, inv = _pack_nibbles(q), (1.0 / s if s is not None else None)
+            if s is not None:
+                self.register_buffer("inv_act_scale", inv.contiguous())
+            else:
+                self.inv_act_scale = None
+            self.register_buffer("nibbles", nib)  # [out, in / 2]
+            self.register_buffer("g_scale", g_scale.contiguous())  # [out, groups]
+            self.register_buffer("g_zero", g_zero.contiguous())
+            # The weight rearranged for the decode-batch matrix-core kernel (not saved: it is a
+            # function of the three buffers above).
+            packed = None
+            gemv = _native("gemv", dev)
+            if gemv is not None and self.in_features % 128 == 0 and group_size % 128 == 0:
+                packed = gemv.int4_gemm_pack(nib, g_scale, g_zero, group_size)
+            self.register_buffer("gemm_packed", packed, persistent=False)
+        self._packed_from = self._stamp()
         self.bias = None
         if linear.bias is not None:
             self.bias = nn.Parameter(linear.bias.detach().to(dev).clone(), requires_grad=False)
@@ -240,10 +243,58 @@ class Int4Linear(nn.Module):
         return _dequant_groups(_unpack_nibbles(self.nibbles), self.g_scale, self.g_zero,
                                self.group_size)
 
+    # gemm_packed is used only while the three buffers are the tensors it was made from, at the
+    # versions they had (_packed_from); calls that find others read the buffers themselves.
+    # Loading a state dict packs again, moving the module keeps the packing.
+
+    def _stamp(self):
+        """(name, tensor, version) of the buffers ``gemm_packed`` stands for; None without a
+        packing, or where a buffer is an inference tensor, whose writes nothing counts."""
+        names = ("nibbles", "g_scale", "g_zero")
+        bufs = [self._buffers.get(n) for n in names]
+        if self.gemm_packed is None or any(t is None or t.is_inference() for t in bufs):
+            return None
+        return tuple((n, weakref.ref(t), t._version) for n, t in zip(names, bufs))
+
+    def _packed_current(self) -> bool:
+        bufs = self._buffers
+        if self._packed_from is None or bufs.get("gemm_packed") is None:
+            return False
+        for name, made_from, version in self._packed_from:
+            t = bufs.get(name)
+            if t is None or made_from() is not t or t._version != version:
+                return False
+        return True
+
+    def _load_from_state_dict(self, *args, **kwargs) -> None:
+        super()._load_from_state_dict(*args, **kwargs)
+        self._packed_from = None
+        bufs = (self.nibbles, self.g_scale, self.g_zero)
+        native = _native("gemv", bufs[0].device)
+        if (self.gemm_packed is not None and native is not None
+                and all(t.is_contiguous() and t.device == self.gemm_packed.device for t in bufs)
+                and [t.dtype for t in bufs] == [torch.uint8, torch.float32, torch.float32]):
+            with torch.inference_mode():  # in place, also where it is an inference tensor
+                self.gemm_packed.copy_(native.int4_gemm_pack(*bufs, self.group_size))
+            self._packed_from = self._stamp()
+
+    def _apply(self, fn, recurse: bool = True):
+        current = self._packed_current()
+        super()._apply(fn, recurse)
+        self._packed_from = self._stamp() if current else None
+        return self
+
+    def __getstate__(self):  # a copy has tensors of its own, at versions of their own
+        return {**self.__dict__, "_packed_from": self._packed_current()}
+
+    def __setstate__(self, state) -> None:
+        super().__setstate__(state)
+        self._packed_from = self._stamp() if state.get("_packed_from", True) else None
+
     def packed_path(self, rows: int) -> bool:
         """``kernel="auto"`` runs the packed matrix-core kernel for ``rows`` activation rows."""
-        return (self.kernel == "auto" and self.gemm_packed is not None
-                and self.gemv_max_rows < rows <= self.max_packed_rows)
+        return (self.kernel == "auto" and self.gemv_max_rows < rows <= self.max_packed_rows
+                and self._packed_current())
 
     def gemm_ok(self) -> bool:
         """Shapes the reference-layout matrix-core kernel (int4_linear_gemm) takes."""
@@ -278,7 +329,7 @@ class Int4Linear(nn.Module):
             return "gemv"
         if x is not None and self._tile_ok(x):
             return "tile"
-        if self.gemm_packed is not None and not self.gemm_ok():
+        if not self.gemm_ok() and self._packed_current():
             return "gemm"
         return "gemm_ref" if self.gemm_ok() else "aten"
 
@@ -291,9 +342,11 @@ class Int4Linear(nn.Module):
             xs = x2 * self.inv_act_scale if self.inv_act_scale is not None else x2
             y = xs @ self.dequantize().t()
         elif path == "gemm":
-            y = native.int4_linear_gemm_packed(x2.contiguous(), self.gemm_packed,
-                                               self.out_features, self.group_size,
-                                               self.inv_act_scale)
+            packed = self.gemm_packed
+            if self.kernel == "gemm" and not self._packed_current():  # "auto" comes here with a current one
+                packed = native.int4_gemm_pack(self.nibbles, self.g_scale, self.g_zero, self.group_size)
+            y = native.int4_linear_gemm_packed(x2.contiguous(), packed, self.out_features,
+                                               self.group_size, self.inv_act_scale)
         elif path == "tile":
             # The call packs the weight itself, from the buffers as they are now: a write to them
             # that no version counter sees (through .data, by a kernel) counts too.

@@ -418,11 +418,11 @@ class QuantCausalLM(nn.Module):
                 h = fo.add_rmsnorm_xfrag_(x, attn, L.post_attention_layernorm,
                                           L.gate_up_proj.inv_act_scale, eps)
                 a = fo.silu_mul_xfrag(gemm(h, L.gate_up_proj, H), L.down_proj.inv_act_scale)
-                to_frag = nxt is not None or self._lm_frag(B)
+                to_frag = nxt is not None or self._head_frag(B)
                 down = gemm_planes(a, L.down_proj, I) if to_frag else gemm(a, L.down_proj, I)
                 if nxt is not None:
                     h = fo.add_rmsnorm_xfrag_(x, down, nxt_w, nxt.qkv_proj.inv_act_scale, eps)
-                elif self._lm_frag(B):
+                elif to_frag:
                     inv = self.lm_head.inv_act_scale if self.lm_head is not None else None
                     h = fo.add_rmsnorm_xfrag_(x, down, nxt_w, inv, eps)
                 else:
@@ -436,9 +436,10 @@ class QuantCausalLM(nn.Module):
     def _lm_frag(self, rows: int) -> bool:
         """The LM head reads the final norm's activation fragments: the int4 head on its packed
         weight, or the fp32 head's split-bf16 matrix-core kernel (``fp32_head_kernel``)."""
+        return self._xfrag_ok(rows) and self._head_frag(rows)
+
+    def _head_frag(self, rows: int) -> bool:
         m = self.lm_head
-        if not self._xfrag_ok(rows):
-            return False
         if m is not None:
             return m.packed_path(rows)
         return self.fp32_head_kernel and self.cfg.hidden_size % 128 == 0

@@ -186,3 +186,40 @@ def test_embed_rmsnorm(gpu):
     ref = ofo.rmsnorm_f64(emb[ids[:4]], w, 1e-6)
     assert np.abs(h[:4] - ref).max() <= 2e-6 * np.abs(ref).max()
     assert np.isnan(x[4:]).all() and np.isnan(h[4:]).all()  # ids outside [0, V)
+
+
+@pytest.mark.parametrize("rows", [1, 8, 40])
+def test_decode_follows_a_loaded_state_dict(gpu, rows):
+    """The step, eager and captured before the load, runs the weights that the model holds now."""
+    from llmserve.kv_cache import KVCache
+    from llmserve.model_runner import DecodeRunner
+    from llmserve.transformer import ModelConfig, QuantCausalLM
+
+    cfg = ModelConfig(vocab_size=512, hidden_size=256, intermediate_size=512, num_hidden_layers=2,
+                      num_attention_heads=4, num_key_value_heads=2, head_dim=128,
+                      max_position_embeddings=2048)
+    a, b = (QuantCausalLM(cfg, 128, quantize_lm_head=True, seed=s) for s in (1, 2))
+    ids = torch.arange(rows, device="cuda")
+    ctx = torch.full((rows,), 5, device="cuda")
+    tables = torch.arange(rows, device="cuda").view(rows, 1)
+
+    def runner(m):
+        return DecodeRunner(m, KVCache(cfg, rows, 16, device="cuda", kv_dtype="int8"), ids, ctx, tables)
+
+    ra, rb = runner(a), runner(b)
+    ra.capture()
+    assert a._xfrag_ok(rows) == (rows > 4)
+    a.load_state_dict(b.state_dict())
+    want = rb.forward_logits()
+    assert torch.equal(ra.forward_logits(), want)
+    ra.replay()
+    assert torch.equal(ra.logits, want)
+    ra.restore((ids, ctx, [(k.data, k.scale, v.data, v.scale) for k, v in ra.cache.layers]))
+    a.layers[1].down_proj.g_scale.mul_(2)  # the fragments' packed weights no longer hold
+    b.layers[1].down_proj.g_scale.mul_(2)
+    assert not a._xfrag_ok(rows)
+    got, want = ra.forward_logits(), rb.forward_logits()
+    assert torch.equal(got, want)
+    b.fuse_xfrag = False
+    rb.model.layers[1].down_proj.kernel = "gemv" if rows <= 16 else "auto"
+    assert (rb.forward_logits() - want).norm() <= 1e-3 * want.norm()

@@ -445,3 +445,81 @@ def test_reference_binding_from_integration_doc(tmp_path, case):
                        capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and "binding ok" in r.stdout, r.stderr[-3000:]
     assert "RecursionError" not in r.stderr
+
+
+def _plain_int4_ops():
+    """The int4 ops Int4Linear calls, as torch code: the packed weight holds copies of its buffers."""
+    from llmserve.quant import _dequant_groups, _unpack_nibbles
+
+    def dense(nib, gs, gz, group):
+        return _dequant_groups(_unpack_nibbles(nib), gs, gz, group)
+
+    def product(x, nib, gs, gz, group, inv=None, packed=None):
+        return (x if inv is None else x * inv) @ dense(nib, gs, gz, group).t()
+
+    def pack(nib, gs, gz, group):
+        return dense(nib, gs, gz, group).flatten().view(torch.uint8).clone()
+
+    def packed_product(x, packed, n, group, inv=None):
+        return (x if inv is None else x * inv) @ packed.view(torch.float32).view(n, -1).t()
+
+    return SimpleNamespace(int4_linear=product, int4_linear_gemm=product, int4_linear_tile=product,
+                           int4_gemm_pack=pack, int4_linear_gemm_packed=packed_product)
+
+
+@pytest.mark.parametrize("built_in_inference_mode", [False, True])
+def test_packed_int4_weight_follows_its_buffers(monkeypatch, built_in_inference_mode):
+    """Every route reads the weight the module holds now, whatever changed it; a loaded state dict is
+    packed again (into the same memory), a moved or copied module keeps its packing."""
+    import copy
+    import io
+
+    from llmserve import quant
+    from llmserve.quant import Int4Linear
+
+    ops = _plain_int4_ops()
+    monkeypatch.setattr(quant, "_native", lambda kind, dev: ops if kind == "gemv" else None)
+    with torch.inference_mode(built_in_inference_mode):
+        a, b = (Int4Linear(_linear(24, 256, s), 128) for s in (1, 2))
+
+    def right(m, packed):
+        assert m.packed_path(64) == packed
+        for rows in (1, 8, 64, 300):
+            x = torch.randn(rows, 256, generator=torch.Generator().manual_seed(rows))
+            for kernel in ("auto", "gemm") if rows == 64 else ("auto",):
+                m.kernel = kernel
+                with torch.no_grad():
+                    y = m(x)
+                    ref = x @ m.dequantize().t()
+                del m.kernel
+                assert torch.allclose(y, ref, atol=1e-4), (rows, kernel)
+
+    right(a, True)
+    at = a.gemm_packed.data_ptr()
+    a.load_state_dict(b.state_dict())
+    right(a, True)
+    assert a.gemm_packed.data_ptr() == at
+    x = torch.ones(64, 256)
+    with torch.no_grad():  # another module's tensors for one call
+        other = {k: v * 2 for k, v in b.state_dict().items() if k != "nibbles"}
+        y = torch.func.functional_call(a, other, (x,))
+        assert torch.allclose(y, 2 * a(x), atol=1e-4)
+    right(a, True)
+    right(copy.deepcopy(a), True)
+    buf = io.BytesIO()
+    torch.save(a, buf)
+    buf.seek(0)
+    right(torch.load(buf, weights_only=False), True)
+    right(a.to(torch.float32), True)
+    a.g_scale.mul_(2)
+    right(a, False)
+    right(copy.deepcopy(a), False)
+    a.load_state_dict(b.state_dict(), assign=True)
+    right(a, True)
+    a.g_zero = a.g_zero + 1
+    right(a, False)
+    a.load_state_dict({k: v.clone() for k, v in b.state_dict().items()})
+    right(a, True)
+    with torch.inference_mode():
+        a.g_scale.mul_(2)
+    right(a, False)
