@@ -271,6 +271,35 @@ at::Tensor int4_linear_tile_meta(const at::Tensor& x, const at::Tensor& nibbles,
   return at::empty_symint({x.sym_size(0), nibbles.sym_size(0)}, x.options());
 }
 
+// int4_linear_tile as torch ops (dequantize, then matmul): where the call is differentiated or
+// batched over, also through transforms that the caller cannot see on its tensors.
+at::Tensor int4_linear_tile_torch(const at::Tensor& x, const at::Tensor& nibbles, const at::Tensor& scale,
+                                  const at::Tensor& zero, int64_t group_size,
+                                  const std::optional<at::Tensor>& inv_act_scale,
+                                  const std::optional<at::Tensor>& packed) {
+  const at::Tensor q = at::stack({at::bitwise_and(nibbles, 15), at::bitwise_right_shift(nibbles, 4)}, -1)
+                           .flatten(1)
+                           .unflatten(1, at::IntArrayRef({-1, group_size}))
+                           .to(at::kFloat);
+  const at::Tensor w = ((q - 8) * scale.unsqueeze(-1) + zero.unsqueeze(-1)).flatten(1);
+  return at::matmul(inv_act_scale.has_value() ? x * *inv_act_scale : x, w.t());
+}
+
+at::Tensor int4_linear_tile_autograd(const at::Tensor& x, const at::Tensor& nibbles, const at::Tensor& scale,
+                                     const at::Tensor& zero, int64_t group_size,
+                                     const std::optional<at::Tensor>& inv_act_scale,
+                                     const std::optional<at::Tensor>& packed) {
+  bool differentiated = false;
+  for (const at::Tensor* t : {&x, &scale, &zero, inv_act_scale.has_value() ? &*inv_act_scale : &x})
+    differentiated |= (at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(0).defined();
+  if (differentiated) return int4_linear_tile_torch(x, nibbles, scale, zero, group_size, inv_act_scale, packed);
+  const at::AutoDispatchBelowADInplaceOrView below;
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("llmserve_hip::int4_linear_tile", "")
+                             .typed<decltype(int4_linear_tile)>();
+  return op.call(x, nibbles, scale, zero, group_size, inv_act_scale, packed);
+}
+
 at::Tensor int4_gemm_pack(const at::Tensor& nibbles, const at::Tensor& scale,
                           const at::Tensor& zero, int64_t group_size) {
   TORCH_CHECK(nibbles.scalar_type() == at::kByte && scale.scalar_type() == at::kFloat &&
@@ -1010,3 +1039,6 @@ TORCH_LIBRARY_IMPL(llmserve_hip, CUDA, m) {
 
 // Shapes for tracing (torch.compile, FakeTensor).
 TORCH_LIBRARY_IMPL(llmserve_hip, Meta, m) { m.impl("int4_linear_tile", &int4_linear_tile_meta); }
+
+TORCH_LIBRARY_IMPL(llmserve_hip, Autograd, m) { m.impl("int4_linear_tile", &int4_linear_tile_autograd); }
+TORCH_LIBRARY_IMPL(llmserve_hip, FuncTorchBatched, m) { m.impl("int4_linear_tile", &int4_linear_tile_torch); }

@@ -303,15 +303,16 @@ class Int4Linear(nn.Module):
 
     def _tile_ok(self, x: torch.Tensor) -> bool:
         """Inputs the tiled GEMM (int4_linear_tile) takes; the others keep the torch ops, which
-        differentiate (also through the scales), promote types and follow autocast."""
+        differentiate (also through the scales), promote types and follow autocast. (Forward-mode
+        derivatives, and gradients outside of a vmap, which the tensors here don't show, are the
+        op's own: it runs as torch ops under them.)"""
         rows, (n, k) = x.shape[0], (self.out_features, self.in_features)
         return (k % 128 == 0 and self.group_size % 64 == 0 and x.dtype == torch.float32
                 and rows < 2**24 and n < 2**22 and k < 2**20 and rows * k < 2**36
                 and not (torch.is_grad_enabled() and any(
                     t is not None and t.requires_grad
                     for t in (x, self.g_scale, self.g_zero, self.inv_act_scale)))
-                and not torch.is_autocast_enabled(x.device.type)
-                and torch.autograd.forward_ad._current_level < 0)
+                and not torch.is_autocast_enabled(x.device.type))
 
     def _path(self, rows: int, native, x: torch.Tensor | None = None) -> str:
         if self.kernel not in ("auto", "gemv", "gemm", "gemm_ref", "aten"):

@@ -175,3 +175,16 @@ def test_large_batches_follow_the_buffers(gpu, group, rows):
     assert follows(a, x)
     a.nibbles = torch.flip(a.nibbles, (0,)).contiguous()
     assert follows(a, x)
+
+
+def test_transforms_through_the_module(gpu):
+    """A forward-mode derivative, and a gradient taken outside of a vmap (which no tensor inside shows)."""
+    from llmserve.quant import Int4Linear
+
+    m = Int4Linear(torch.nn.Linear(256, 40, bias=False, device="cuda"), 64)
+    w = m.dequantize()
+    x, dx = torch.randn(2, 3, 33, 256, device="cuda")
+    _, t = torch.func.jvp(m, (x[0],), (dx[0],))
+    assert (t - dx[0] @ w.t()).norm() <= 1e-5 * t.norm()
+    g = torch.func.grad(lambda x: torch.vmap(m)(x).square().sum())(x)
+    assert (g - 2 * (x @ w.t()) @ w).norm() <= 1e-5 * g.norm()

@@ -523,3 +523,55 @@ def test_packed_int4_weight_follows_its_buffers(monkeypatch, built_in_inference_
     with torch.inference_mode():
         a.g_scale.mul_(2)
     right(a, False)
+
+
+def test_int4_tile_op_under_transforms():
+    """int4_linear_tile differentiates and batches as the torch ops it stands for, in every nesting (a
+    gradient taken outside of a vmap shows on none of the tensors inside it)."""
+    from llmserve import _native
+    from llmserve.quant import Int4Linear
+
+    try:
+        op = _native.ops().int4_linear_tile
+    except (OSError, RuntimeError, FileNotFoundError) as e:
+        pytest.skip(f"op library: {e}")
+    plain = _plain_int4_ops().int4_linear_tile
+    calls = []
+
+    def kernel(x, nib, gs, gz, group, inv=None, packed=None):
+        calls.append(x.shape)
+        return plain(x, nib, gs, gz, group, inv)
+
+    lib = torch.library.Library("llmserve_hip", "IMPL")
+    try:
+        lib.impl("int4_linear_tile", kernel, "CPU")  # stands in for the HIP kernel
+        m = Int4Linear(_linear(6, 128, 3), 64, torch.rand(128) + 0.5)
+        x, dx = (torch.randn(3, 5, 128, generator=torch.Generator().manual_seed(s)) for s in (1, 2))
+
+        def run(f):
+            def lin(x, gs=m.g_scale):
+                return f(x, m.nibbles, gs, m.g_zero, 64, m.inv_act_scale)
+
+            def loss(x):
+                return lin(x).square().sum()
+
+            fn = torch.func
+            return [lin(x[0]), fn.grad(loss)(x[0]), fn.vmap(lin)(x), fn.vmap(fn.grad(loss))(x),
+                    fn.grad(lambda x: fn.vmap(lin)(x).square().sum())(x), fn.jvp(lin, (x[0],), (dx[0],))[1],
+                    fn.jvp(fn.vmap(lin), (x,), (dx,))[1], fn.vmap(lambda gs: lin(x[0], gs))(m.g_scale * dx[:, 0, :1, None]),
+                    fn.grad(lambda gs: lin(x[0], gs).square().sum())(m.g_scale),
+                    fn.vmap(fn.jacrev(lin))(x)]
+
+        for got, want in zip(run(op), run(plain), strict=True):
+            assert got.shape == want.shape and (got - want).norm() <= 1e-5 * want.norm()
+        calls.clear()
+        with torch.inference_mode():
+            op(x[0], m.nibbles, m.g_scale, m.g_zero, 64)
+        with torch.no_grad():
+            op(x[0].clone().requires_grad_(), m.nibbles, m.g_scale, m.g_zero, 64)
+        op(x[0], m.nibbles, m.g_scale, m.g_zero, 64)
+        assert len(calls) == 3  # the kernel, wherever nothing is differentiated
+        y = op(x[0].clone().requires_grad_(), m.nibbles, m.g_scale, m.g_zero, 64)
+        assert y.requires_grad and len(calls) == 3
+    finally:
+        lib._destroy()
