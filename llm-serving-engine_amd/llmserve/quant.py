@@ -307,11 +307,12 @@ class Int4Linear(nn.Module):
         derivatives, and gradients outside of a vmap, which the tensors here don't show, are the
         op's own: it runs as torch ops under them.)"""
         rows, (n, k) = x.shape[0], (self.out_features, self.in_features)
+        scales = [t for t in (self.g_scale, self.g_zero, self.inv_act_scale) if t is not None]
         return (k % 128 == 0 and self.group_size % 64 == 0 and x.dtype == torch.float32
                 and rows < 2**24 and n < 2**22 and k < 2**20 and rows * k < 2**36
-                and not (torch.is_grad_enabled() and any(
-                    t is not None and t.requires_grad
-                    for t in (x, self.g_scale, self.g_zero, self.inv_act_scale)))
+                and self.nibbles.is_contiguous()
+                and all(t.dtype == torch.float32 and t.is_contiguous() for t in scales)
+                and not (torch.is_grad_enabled() and any(t.requires_grad for t in (x, *scales)))
                 and not torch.is_autocast_enabled(x.device.type))
 
     def _path(self, rows: int, native, x: torch.Tensor | None = None) -> str:

@@ -188,3 +188,21 @@ def test_transforms_through_the_module(gpu):
     assert (t - dx[0] @ w.t()).norm() <= 1e-5 * t.norm()
     g = torch.func.grad(lambda x: torch.vmap(m)(x).square().sum())(x)
     assert (g - 2 * (x @ w.t()) @ w).norm() <= 1e-5 * g.norm()
+
+
+def test_buffers_of_other_types_and_strides_keep_the_torch_ops(gpu):
+    """Scales in 16 bits (a module moved with .half()), and buffers that are views of other memory."""
+    from llmserve.quant import Int4Linear
+
+    lin = torch.nn.Linear(256, 40, bias=False, device="cuda")
+    act = torch.rand(256, device="cuda") + 0.5
+    x = torch.randn(33, 256, device="cuda")
+    m = Int4Linear(lin, 64, act).half()
+    xs = x * m.inv_act_scale
+    assert torch.equal(m(x), xs @ m.dequantize().t()) and m(x).dtype == torch.float32
+    for name in ("nibbles", "g_scale", "g_zero", "inv_act_scale"):
+        m = Int4Linear(lin, 64, act)
+        y = m(x)
+        t = getattr(m, name)
+        setattr(m, name, t.repeat_interleave(2, -1)[..., ::2])
+        assert (m(x) - y).norm() <= 2e-6 * y.norm()
