@@ -67,7 +67,7 @@ __host__ __device__ inline int64_t sum_steps(int64_t units) { return (units + 31
 
 // The workspace of a call.
 struct SplitOut {
-  float* rscale;   // [mp] 2^-e of each row
+  float* rscale;   // [mp] 2^-e of each row; negative: the split pass has written the row of y
   _Float16* xf;    // [row tile][block][q][piece][lane][8]
   // int4:
   _Float16* xs;    // [row tile][step of 32 units][hi, lo][lane][8]: unit sums of x' 2^e, scaled by 2^-8
@@ -191,12 +191,32 @@ __device__ __forceinline__ void pack_block(const SplitOut& o, const WeightIn& in
   }
 }
 
+// A row of x' with an infinity: y as float32 arithmetic on the dequantized weight has it (signed
+// infinities; NaN where opposite ones meet or the weight is 0). Two pieces, or the sums' split into
+// codes and zero term, would give NaN everywhere. No load of the usual rows passes here.
+__device__ __forceinline__ void plain_row(const float* x, const float* inv, const WeightIn& in, float* y, int K) {
+  const int G = K / in.group;
+  for (int n = threadIdx.x % kWave; n < in.N; n += kWave) {
+    const uint8_t* row = in.nib + static_cast<int64_t>(n) * (K / 2);
+    float sum = 0.f;
+    for (int g = 0; g < G; ++g) {
+      const float s = in.gs[static_cast<int64_t>(n) * G + g], z = in.gz[static_cast<int64_t>(n) * G + g];
+      for (int k = g * in.group; k < (g + 1) * in.group; ++k) {
+        const int q = row[k / 2] >> (k % 2 * 4) & 15;
+        const float w = __fadd_rn(__fmul_rn(static_cast<float>(q - 8), s), z);
+        sum = __builtin_fmaf(inv ? __fmul_rn(x[k], inv[k]) : x[k], w, sum);
+      }
+    }
+    y[n] = sum;
+  }
+}
+
 // One wavefront per row of x (and of the padding); then, for int4, one per 16-channel tile of
 // the zero term and, for a weight in the reference layout, one per packed (slab, block).
 template <Order O>
 __global__ __launch_bounds__(kSplitRows* kWave) void split_rows_kernel(
     const float* __restrict__ x, const float* __restrict__ inv, SplitOut o, int M, int K, int mp, int nblk,
-    WeightIn in) {
+    WeightIn in, float* __restrict__ y) {
   constexpr int P = pieces(O);
   const int lane = threadIdx.x % kWave;
   const int m = blockIdx.x * kSplitRows + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
@@ -255,7 +275,8 @@ __global__ __launch_bounds__(kSplitRows* kWave) void split_rows_kernel(
   // the power of two that brings the row's largest value to [2^14, 2^15)
   const int ex = exponent_to_15(top);
   const float up = m < M ? __builtin_amdgcn_ldexpf(1.f, ex) : 0.f;
-  if (lane == 0) o.rscale[m] = __builtin_amdgcn_ldexpf(1.f, -ex);
+  const bool plain = O != kInt8 && top == __builtin_inff();  // uniform; the GEMM leaves such a row alone
+  if (lane == 0) o.rscale[m] = plain ? -1.f : __builtin_amdgcn_ldexpf(1.f, -ex);
 
   const int mt = m / 16, fr = m % 16;
   const int units = K / unit(O);
@@ -309,6 +330,7 @@ __global__ __launch_bounds__(kSplitRows* kWave) void split_rows_kernel(
   if constexpr (O != kInt8) {
     const int padded = static_cast<int>(sum_steps(units)) * 32;
     for (int u = units + lane; u < padded; u += kWave) store_sum(u, 0.f);
+    if (plain) plain_row(xr, inv, in, y + static_cast<int64_t>(m) * in.N, K);
   }
 }
 
@@ -615,11 +637,12 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_tile_kernel(TileArgs a)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int row = 16 * t + 4 * fc + e;
+      const bool on = m0 + row < a.M && (O == kInt8 || rm[t][e] > 0.f);
       const uint32_t row_ofs = static_cast<uint32_t>(row) * static_cast<uint32_t>(a.N) * 4;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int n = n0 + 16 * u + fr;
-        const uint32_t ofs = n < a.N && m0 + row < a.M ? row_ofs + static_cast<uint32_t>(n) * 4 : 0x80000000u;
+        const uint32_t ofs = n < a.N && on ? row_ofs + static_cast<uint32_t>(n) * 4 : 0x80000000u;
         const float v = O == kInt8 ? acc[t][u][e] * cs[u] : acc[t][u][e];
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v * rm[t][e]), ry, ofs, 0, 0);
       }
@@ -659,7 +682,7 @@ void launch_tile(const float* x, const float* inv, const WeightIn& in, TileArgs 
   int64_t waves = mp;
   if (O != kInt8) waves += slabs_of(a.N) * (4 + (in.packed ? 0 : a.K / kBlk));
   lsh::launch(split_rows_kernel<O>, dim3(static_cast<unsigned>((waves + kSplitRows - 1) / kSplitRows)),
-              dim3(kSplitRows * kWave), 0, st, false, x, inv, a.a, a.M, a.K, mp, a.blocks, in);
+              dim3(kSplitRows * kWave), 0, st, false, x, inv, a.a, a.M, a.K, mp, a.blocks, in, a.y);
   a.tiles_m = (a.M + 16 * TM - 1) / (16 * TM);
   a.tiles_n = (a.N + 64 * WN - 1) / (64 * WN);
   const int64_t total = static_cast<int64_t>(a.tiles_m) * a.tiles_n;

@@ -206,3 +206,29 @@ def test_buffers_of_other_types_and_strides_keep_the_torch_ops(gpu):
         t = getattr(m, name)
         setattr(m, name, t.repeat_interleave(2, -1)[..., ::2])
         assert (m(x) - y).norm() <= 2e-6 * y.norm()
+
+
+@pytest.mark.parametrize("M,N,K,group,packed", [(40, 96, 256, 64, False), (129, 1000, 384, 128, True),
+                                                (300, 12300, 128, 64, False)])
+def test_infinities_keep_their_signs(gpu, M, N, K, group, packed):
+    """A row with infinities is what arithmetic on the dequantized weight gives: signed infinities, NaN
+    where opposite ones meet or the weight is 0; the other rows are as they were."""
+    x, nib, gs, gz, inv = make(M + K, M, N, K, group, True)
+    clean = run(x, nib, gs, gz, group, inv, packed)[0]
+    gz[3, 0], gs[5, 0] = 0, 0  # code 8 of channel 3 is a weight of 0
+    nib[3, 0], gz[5, 0] = 0x88, 0
+    bad = {1: {0: np.inf}, 2: {7: -np.inf}, M - 1: {1: np.inf, K - 1: np.inf}, 9: {3: np.inf, 5: np.nan}}
+    for r, where in bad.items():
+        for k, v in where.items():
+            x[r, k] = v
+    x[4, 2] = 3e38  # an infinity from the AWQ product
+    inv[2] = 4
+    rows = sorted([*bad, 4])
+    y = run(x, nib, gs, gz, group, inv, packed)[0].cpu().numpy()
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = mr.int4_linear_f64(x[rows], nib, gs, gz, group, inv)
+    assert not np.isfinite(want).any() and np.isinf(want[0]).any()
+    np.testing.assert_array_equal(y[rows], want.astype(F32))
+    fine = [r for r in range(M) if r not in rows]
+    ref = mr.int4_linear_f64(x[fine], nib, gs, gz, group, inv)
+    assert np.linalg.norm(y[fine] - ref) <= 2e-6 * np.linalg.norm(ref)
