@@ -54,9 +54,9 @@ constexpr float kLog2e = 1.4426950408889634f;
 // float64 error over the fp32 cache 2.2e-7 instead of 1.6e-7).
 constexpr float kLazy = 4.f;
 constexpr int kTop = 11, kUpMin = -5, kUpMax = 23;
-// A v scale that is not finite is staged as kHuge, so that a weight of 0 (a token that the query does
-// not see) times it stays 0; a weight that is not 0 still overflows fp16, as the reference follows
-// staged v scales up to 2^(kTop + kMaxLv) only (scales of 2^88 at least), and the output is NaN.
+// A v scale that is not finite (or too large to stage) is staged as kHuge, so that a weight of 0 (a token
+// that the query does not see) times it stays 0. The queries that see one are computed again, row by
+// row (plain_chunk), and so are those whose scores were not finite.
 constexpr float kHuge = 3.402823466e38f, kMaxLv = 100.f;
 
 struct PrefillArgs {
@@ -154,6 +154,80 @@ __device__ __forceinline__ void read_ahead() {
     __builtin_amdgcn_sched_group_barrier(kRead, PL, 0);
   }
   __builtin_amdgcn_sched_group_barrier(kMfma, kAhead * M, 0);
+}
+
+// A chunk for the queries (bits of `redo`) that see a value row (fp32: also a key row) that is not
+// finite, as float32 arithmetic row by row has it: an infinity stays in its channel, a score of
+// -infinity is a weight of 0. The pieces of such a row would give NaN in every channel, or miss the
+// row where its weight is small. Each wavefront takes its 16 query tokens, 4 at a time, lanes over the
+// dims; `put` gets (query token, head of the pair, reference, sum, this lane's dims lane + 64 i).
+template <typename E, int D, typename Put>
+__device__ __forceinline__ void plain_chunk(const PrefillArgs& a, int kvh, int g0, int row0, int rows, int sees,
+                                            int k0, int k1, const uint32_t (&redo)[kHeads], const int64_t* bt,
+                                            Put put) {
+  constexpr int kTok = 4, N = kTok * kHeads, W = D / kWave;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  for (int i0 = 0; i0 < 16; i0 += kTok) {
+    float q[N][W], m[N], l[N], acc[N][W];
+    uint32_t on = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int i = 16 * wave + i0 + j / kHeads;
+      const int64_t head = kvh * a.G + min(g0 + j % kHeads, a.G - 1), tok = row0 + min(i, rows - 1);
+      m[j] = -1e30f;
+      l[j] = 0.f;
+      bool finite = true;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const int d = lane + kWave * w;
+        float v = a.q[(tok * a.Hq + head) * D + d];
+        if (a.q_mult) v = __fmul_rn(v, a.q_mult[head * D + d]);
+        finite &= fabsf(v) < __builtin_inff();
+        q[j][w] = v * (a.scale * kLog2e);
+        acc[j][w] = 0.f;
+      }
+      if ((redo[j % kHeads] >> (i0 + j / kHeads) & 1) && i < rows && g0 + j % kHeads < a.G) {
+        on |= 1u << j;
+        if (__ballot(!finite) != 0) l[j] = __builtin_nanf("");  // NaN whatever the cache holds
+      }
+    }
+    uint32_t todo = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) todo |= (on >> j & 1) && l[j] == 0.f ? 1u << j : 0u;
+    for (int t = k0; t < k1 && todo != 0; ++t) {
+      const int block = a.bs_shift >= 0 ? t >> a.bs_shift : t / a.bs;
+      const int64_t id = bt[block];
+      if (id < 0 || id >= a.num_slots / a.bs) continue;
+      const int64_t at = (id * a.bs + (t - block * a.bs)) * a.Hk + kvh;
+      float k[W], v[W], ks = 1.f, vs = 1.f;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        k[w] = static_cast<float>(static_cast<const E*>(a.kc)[at * D + lane + kWave * w]);
+        v[w] = static_cast<float>(static_cast<const E*>(a.vc)[at * D + lane + kWave * w]);
+      }
+      if constexpr (std::is_same_v<E, int8_t>) {
+        ks = a.ks[at];
+        vs = a.vs[at];
+      }
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        if (!(todo >> j & 1) || t >= sees + 16 * wave + i0 + j / kHeads) continue;
+        float s = q[j][0] * k[0];
+#pragma unroll
+        for (int w = 1; w < W; ++w) s = __builtin_fmaf(q[j][w], k[w], s);
+        s = lsh::group_sum<kWave>(s) * ks;
+        const float top = fmaxf(m[j], s), f = __builtin_amdgcn_exp2f(m[j] - top);
+        const float p = __builtin_amdgcn_exp2f(s - top);
+        m[j] = top;
+        l[j] = l[j] * f + p;
+#pragma unroll
+        for (int w = 0; w < W; ++w) acc[j][w] = __builtin_fmaf(p * vs, v[w], acc[j][w] * f);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (on >> j & 1) put(16 * wave + i0 + j / kHeads, j % kHeads, m[j], l[j], acc[j]);
+  }
 }
 
 template <typename E, int D>
@@ -413,6 +487,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
     for (int d = 0; d < DT; ++d) acc[c][d] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const int limit = sees + tok;  // tokens this lane's query sees
+  uint64_t huge = 0;             // lanes that see a v scale staged as kHuge
 
   int slot = slot_of(0, fetch_id(0));
   load(slot);
@@ -496,6 +571,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
         }
       }
     }
+    huge |= __ballot(vtop >= kHuge);
     const float lv = fminf(fmaxf(__builtin_amdgcn_logf(max_over_fc(vtop)) - kTop, -kMaxLv), kMaxLv);
     float top[kHeads];
     bool raise = false;
@@ -584,10 +660,17 @@ if constexpr (PL == 1) {
 
   // ---- output: lane (fr, fc) holds dims 16 d + 4 fc + e of its query -----------------------------
   const bool whole = size >= ctx;
+  auto part_at = [&](int tok, int c) {
+    return (((static_cast<int64_t>(tile) * a.Hk * a.pairs + hp) * a.splits + chunk) * kHeads + c) * kQT + tok;
+  };
+  huge |= huge >> 32;
+  huge |= huge >> 16;
+  uint32_t redo[kHeads];  // bits: this wavefront's query tokens
 #pragma unroll
   for (int c = 0; c < kHeads; ++c) {
     const float l = sum_over_fc(sum[c]);
-    if (16 * wave + fr >= rows || g0 + c >= a.G) continue;
+    redo[c] = static_cast<uint32_t>(huge | __ballot(l != l)) & 0xffffu;
+    if (16 * wave + fr >= rows || (redo[c] >> fr & 1) || g0 + c >= a.G) continue;
     if (whole) {
       const float inv = 1.f / (l * v_up);
       float* o = a.out + (static_cast<int64_t>(row0 + tok) * a.Hq + head[c]) * D + 4 * fc;
@@ -595,7 +678,7 @@ if constexpr (PL == 1) {
       for (int d = 0; d < DT; ++d)
         *reinterpret_cast<f32x4*>(o + 16 * d) = acc[c][d] * inv;
     } else {
-      const int64_t at = (((static_cast<int64_t>(tile) * a.Hk * a.pairs + hp) * a.splits + chunk) * kHeads + c) * kQT + tok;
+      const int64_t at = part_at(tok, c);
       float* o = a.part_acc + at * D + 4 * fc;
 #pragma unroll
       for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4*>(o + 16 * d) = acc[c][d] * (1.f / v_up);
@@ -604,6 +687,24 @@ if constexpr (PL == 1) {
         a.part_rl[2 * at + 1] = l;
       }
     }
+  }
+  if (redo[0] | redo[1]) {
+    plain_chunk<E, D>(a, kvh, g0, row0, rows, sees, k0, k1, redo, bt,
+                      [&](int t, int c, float m, float l, const float (&v)[D / kWave]) {
+                        const int64_t at = part_at(t, c);
+                        float* o = a.out + (static_cast<int64_t>(row0 + t) * a.Hq + kvh * a.G + g0 + c) * D;
+#pragma unroll
+                        for (int i = 0; i < D / kWave; ++i) {
+                          if (whole)
+                            o[lane + kWave * i] = v[i] / l;
+                          else
+                            a.part_acc[at * D + lane + kWave * i] = v[i];
+                        }
+                        if (!whole && lane == 0) {
+                          a.part_rl[2 * at] = m;
+                          a.part_rl[2 * at + 1] = l;
+                        }
+                      });
   }
 }
 

@@ -153,3 +153,35 @@ def test_dispatch(gpu, monkeypatch):
     with pytest.raises(RuntimeError, match="tile 0 outside"):  # more tokens than the batch has
         ops.paged_attention_prefill_(torch.empty_like(q), q, k, k, None, None, meta.block_tables,
                                      meta.prefill_tiles, meta.prefill_tiles_host, 16, 1.0)
+
+
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("q_lens,ctx,geom", [([100], [100], (4, 2, 64, 16)), ([70, 1], [1500, 30], (3, 1, 128, 16))])
+def test_infinities_stay_where_they_are(gpu, int8, q_lens, ctx, geom):
+    """An infinite value reaches its own channel only, an infinite key the tokens it scores +inf or NaN
+    (-inf is a weight of 0), an infinite value scale the channels whose code is not 0, also where
+    the weight is small (down to e^-40), over one chunk and several: as float64 has it."""
+    q, k, v, tables, meta, dev, mult = make(9, q_lens, ctx, geom, int8)
+    n, inf = ctx[0], np.inf
+    a, b, c = (tables[0][t // 16] * 16 + t % 16 for t in (n - 90, n - 40, n - 3))
+    if int8:
+        kq, vq, ks, vs = (t.cpu().numpy() for t in dev)
+        vs[[a, b], 0], ks[b, 0], vq[a, 0, 5] = inf, 12 * ks[b, 0], 0
+        with np.errstate(invalid="ignore"):
+            k, v = mr.kv_dequantize(kq, ks), mr.kv_dequantize(vq, vs)
+        host = kq, vq, ks, vs
+    else:
+        v[a, 0, 7], v[b, 0, 9], k[c, 0, 11] = inf, -inf, inf
+        k[b] *= 12
+        host = k, v, None, None
+    for t, h in zip(dev, host):
+        if t is not None:
+            t.copy_(torch.from_numpy(h))
+    got = run(q, meta, dev, mult, geom[2]).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        want = reference(q, k, v, q_lens, ctx, tables, geom, mult)
+    fine = np.isfinite(want)
+    np.testing.assert_array_equal(got[~fine], want[~fine].astype(F32))
+    assert np.linalg.norm(got[fine] - want[fine]) <= 2e-6 * np.linalg.norm(want[fine])
+    last = want[q_lens[0] - 2: q_lens[0], : geom[0] // geom[1]]
+    assert np.isinf(want).any() and (int8 or (np.isfinite(last).any() and np.isnan(last).any()))
