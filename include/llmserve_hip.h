@@ -428,7 +428,8 @@ int llmserve_paged_attention_decode(const float* q, const float* k_cache, const 
  * tile sees i more tokens than its first. `tiles` is in device memory, `tiles_host` the same
  * values on the host (checked against the batch, and the launch is planned from them). int8
  * caches with scales, or float32 caches with k_scale = v_scale = NULL. D = 64 or 128; q, caches and
- * out 16-byte aligned. Query rows outside the tiles are left alone.
+ * out 16-byte aligned. Query rows outside the tiles are left alone. Long contexts are split into chunks,
+ * whose partial results are the workspace: at most 128 MB (tiles in order of falling context take least).
  */
 int64_t llmserve_paged_attention_prefill_workspace_bytes(const int64_t* tiles_host,
                                                          int64_t n_tiles, int64_t Hq, int64_t Hk,

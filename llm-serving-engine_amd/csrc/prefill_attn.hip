@@ -44,6 +44,7 @@ constexpr int kQT = 64;         // query tokens of a tile: 16 per wavefront
 constexpr int kHeads = 2;       // query heads of a workgroup (of one kv head)
 constexpr int kWaves = 4;
 constexpr int kFrag = 1024;     // bytes of a fragment: 64 lanes x 8 fp16
+constexpr int kMaxSplits = 64;  // chunks of a tile: one per lane in the search for a workgroup's chunk
 constexpr float kLog2e = 1.4426950408889634f;
 // Weights: p = exp2(score - ref), ref the running max of score + log2(v scale) (so that p v_scale
 // stays below 2^kLazy: the reference moves only past that), times v_scale 2^up, which brings the fp16
@@ -69,14 +70,58 @@ struct PrefillArgs {
   const int64_t* tiles;  // [n][4]: first query row, query rows, tokens the first row sees, table row
   const float* q_mult;
   float* out;
-  float* part_acc;  // [tile][kv head, head pair][chunk][kHeads][kQT][D]
-  float* part_rl;   // [tile][kv head, head pair][chunk][kHeads][kQT][2] (reference, sum)
+  float* part_acc;  // [chunk of a split tile (part_index)][kv head, head pair][kHeads][kQT][D]
+  float* part_rl;   // ... [kHeads][kQT][2] (reference, sum)
   int64_t num_slots;
-  int n_tiles, Hq, Hk, G, pairs;  // pairs: head pairs of a kv head
+  int Hq, Hk, G, pairs;  // pairs: head pairs of a kv head
   int max_blocks, bs, bs_shift;
   int chunk, splits;  // most tokens of a context chunk (a multiple of 64), most chunks of a tile
+  int whole;          // tiles, at the end of the list, that are one chunk
   float scale;
+  // Workgroups in order: the first chunks of all tiles, the second chunks of the tiles that have one (the
+  // first so many), ...: start[z] is where the chunks z begin, start[splits] their count.
+  int start[kMaxSplits + 1];
 };
+
+// Tokens of the chunks of a context: as few chunks of at most `most` tokens as cover it, evened out.
+__host__ __device__ inline int chunk_size(int ctx, int most) {
+  const int n = (ctx + most - 1) / most, even = (ctx + n - 1) / n;
+  return (even + 63) / 64 * 64;
+}
+
+// What workgroup `unit` of a head pair computes.
+struct Work {
+  int tile, chunk;
+  int row0, rows, sees, tab;  // the tile
+  int ctx, size;              // tokens its last row sees, tokens of a chunk
+  int k0, k1;                 // the chunk's tokens (none: k0 >= ctx)
+};
+
+__device__ __forceinline__ Work work_of(const PrefillArgs& a, int unit) {
+  Work w;
+  w.tile = unit;
+  w.chunk = 0;
+  if (a.splits > 1) {
+    const int lane = threadIdx.x % kWave, from = a.start[lane + 1];
+    w.chunk = __builtin_popcountll(__ballot(lane + 1 < a.splits && unit >= from));
+    w.tile = unit - a.start[w.chunk];
+  }
+  const int64_t* t = a.tiles + 4 * w.tile;
+  w.row0 = static_cast<int>(t[0]);
+  w.rows = static_cast<int>(t[1]);
+  w.sees = static_cast<int>(t[2]);
+  w.tab = static_cast<int>(t[3]);
+  w.ctx = w.sees + w.rows - 1;
+  w.size = chunk_size(w.ctx, a.chunk);
+  w.k0 = w.chunk * w.size;
+  w.k1 = min(w.ctx, w.k0 + w.size);
+  return w;
+}
+
+// Where a tile's chunk lies among the chunks of split tiles.
+__device__ __forceinline__ int part_index(const PrefillArgs& a, int tile, int z) {
+  return z == 0 ? tile : a.start[z] + tile - a.whole;
+}
 
 __device__ __forceinline__ f16x2 as_h2(uint32_t w) { return __builtin_bit_cast(f16x2, w); }
 __device__ __forceinline__ uint32_t as_u(f16x2 h) { return __builtin_bit_cast(uint32_t, h); }
@@ -124,12 +169,6 @@ __device__ __forceinline__ uint32_t bytes_to_h2(uint32_t w) {
   return as_u(as_h2(__builtin_amdgcn_perm(0x64646464u, w, SEL)) - k);
 }
 
-// Tokens of the chunks of a context: as few chunks of at most `most` tokens as cover it, evened out.
-__host__ __device__ inline int chunk_size(int ctx, int most) {
-  const int n = (ctx + most - 1) / most, even = (ctx + n - 1) / n;
-  return (even + 63) / 64 * 64;
-}
-
 template <typename E>
 struct Geo;
 template <>
@@ -162,9 +201,9 @@ __device__ __forceinline__ void read_ahead() {
 // row where its weight is small. Each wavefront takes its 16 query tokens, 4 at a time, lanes over the
 // dims; `put` gets (query token, head of the pair, reference, sum, this lane's dims lane + 64 i).
 template <typename E, int D, typename Put>
-__device__ __forceinline__ void plain_chunk(const PrefillArgs& a, int kvh, int g0, int row0, int rows, int sees,
-                                            int k0, int k1, const uint32_t (&redo)[kHeads], const int64_t* bt,
-                                            Put put) {
+__device__ __forceinline__ void plain_chunk(const PrefillArgs& a, const Work& u, int kvh, int g0,
+                                            const uint32_t (&redo)[kHeads], Put put) {
+  const int64_t* bt = a.bt + static_cast<int64_t>(u.tab) * a.max_blocks;
   constexpr int kTok = 4, N = kTok * kHeads, W = D / kWave;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   for (int i0 = 0; i0 < 16; i0 += kTok) {
@@ -173,7 +212,7 @@ __device__ __forceinline__ void plain_chunk(const PrefillArgs& a, int kvh, int g
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       const int i = 16 * wave + i0 + j / kHeads;
-      const int64_t head = kvh * a.G + min(g0 + j % kHeads, a.G - 1), tok = row0 + min(i, rows - 1);
+      const int64_t head = kvh * a.G + min(g0 + j % kHeads, a.G - 1), tok = u.row0 + min(i, u.rows - 1);
       m[j] = -1e30f;
       l[j] = 0.f;
       bool finite = true;
@@ -186,7 +225,7 @@ __device__ __forceinline__ void plain_chunk(const PrefillArgs& a, int kvh, int g
         q[j][w] = v * (a.scale * kLog2e);
         acc[j][w] = 0.f;
       }
-      if ((redo[j % kHeads] >> (i0 + j / kHeads) & 1) && i < rows && g0 + j % kHeads < a.G) {
+      if ((redo[j % kHeads] >> (i0 + j / kHeads) & 1) && i < u.rows && g0 + j % kHeads < a.G) {
         on |= 1u << j;
         if (__ballot(!finite) != 0) l[j] = __builtin_nanf("");  // NaN whatever the cache holds
       }
@@ -194,7 +233,7 @@ __device__ __forceinline__ void plain_chunk(const PrefillArgs& a, int kvh, int g
     uint32_t todo = 0;
 #pragma unroll
     for (int j = 0; j < N; ++j) todo |= (on >> j & 1) && l[j] == 0.f ? 1u << j : 0u;
-    for (int t = k0; t < k1 && todo != 0; ++t) {
+    for (int t = u.k0; t < u.k1 && todo != 0; ++t) {
       const int block = a.bs_shift >= 0 ? t >> a.bs_shift : t / a.bs;
       const int64_t id = bt[block];
       if (id < 0 || id >= a.num_slots / a.bs) continue;
@@ -211,7 +250,7 @@ __device__ __forceinline__ void plain_chunk(const PrefillArgs& a, int kvh, int g
       }
 #pragma unroll
       for (int j = 0; j < N; ++j) {
-        if (!(todo >> j & 1) || t >= sees + 16 * wave + i0 + j / kHeads) continue;
+        if (!(todo >> j & 1) || t >= u.sees + 16 * wave + i0 + j / kHeads) continue;
         float s = q[j][0] * k[0];
 #pragma unroll
         for (int w = 1; w < W; ++w) s = __builtin_fmaf(q[j][w], k[w], s);
@@ -251,13 +290,11 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int fr = lane % 16, fc = lane / 16;
   const int hp = blockIdx.x, kvh = hp / a.pairs, g0 = hp % a.pairs * kHeads;
-  const int tile = blockIdx.y, chunk = blockIdx.z;
-  const int row0 = static_cast<int>(a.tiles[4 * tile]), rows = static_cast<int>(a.tiles[4 * tile + 1]);
-  const int sees = static_cast<int>(a.tiles[4 * tile + 2]), tab = static_cast<int>(a.tiles[4 * tile + 3]);
-  const int ctx = sees + rows - 1;  // tokens the tile's last row sees
-  const int size = chunk_size(ctx, a.chunk), k0 = chunk * size;
-  if (k0 >= ctx) return;  // whole workgroup
-  const int k1 = min(ctx, k0 + size);
+  const Work w = work_of(a, blockIdx.y);
+  const int rows = w.rows, sees = w.sees, row0 = w.row0, tab = w.tab, k0 = w.k0, k1 = w.k1;
+  if (k0 >= w.ctx) return;  // whole workgroup
+  const bool whole = w.size >= w.ctx;
+  const int part = part_index(a, w.tile, w.chunk);
   const int n_ct = (k1 - k0 + KT - 1) / KT;
 
   // ---- q: this wavefront's 16 tokens, both heads, as B operands --------------------------------
@@ -357,7 +394,9 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
                                        (__attribute__((address_space(3))) void*)(raw[wave][1] + i * kFrag), 16, 0, 0);
     }
     if constexpr (!kF32) {  // lanes 0 .. TW - 1 K scales, the next TW V scales
-      const float* p = lane < TW ? a.ks : a.vs;
+      const float* const k_scales = a.ks;  // (a choice between the members would load the pointer per lane)
+      const float* const v_scales = a.vs;
+      const float* p = lane < TW ? k_scales : v_scales;
       scale = slot >= 0 ? p[static_cast<int64_t>(slot) * a.Hk + kvh] : 0.f;
     }
   };
@@ -659,9 +698,16 @@ if constexpr (PL == 1) {
   }
 
   // ---- output: lane (fr, fc) holds dims 16 d + 4 fc + e of its query -----------------------------
-  const bool whole = size >= ctx;
+  // The arguments, read again (and the work, where it is needed once more): held since the start, they
+  // would be spilled around the loop.
+  typedef const __attribute__((address_space(4))) PrefillArgs* ArgsPtr;
+  ArgsPtr args = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  int unit = blockIdx.y, pair = blockIdx.x;
+  asm("" : "+s"(args), "+s"(unit), "+s"(pair));
+  const PrefillArgs& b = *(const PrefillArgs*)args;
+  const int kv = pair / b.pairs, g = pair % b.pairs * kHeads;
   auto part_at = [&](int tok, int c) {
-    return (((static_cast<int64_t>(tile) * a.Hk * a.pairs + hp) * a.splits + chunk) * kHeads + c) * kQT + tok;
+    return ((static_cast<int64_t>(part) * b.Hk * b.pairs + pair) * kHeads + c) * kQT + tok;
   };
   huge |= huge >> 32;
   huge |= huge >> 16;
@@ -670,39 +716,39 @@ if constexpr (PL == 1) {
   for (int c = 0; c < kHeads; ++c) {
     const float l = sum_over_fc(sum[c]);
     redo[c] = static_cast<uint32_t>(huge | __ballot(l != l)) & 0xffffu;
-    if (16 * wave + fr >= rows || (redo[c] >> fr & 1) || g0 + c >= a.G) continue;
+    if (16 * wave + fr >= rows || (redo[c] >> fr & 1) || g + c >= b.G) continue;
     if (whole) {
       const float inv = 1.f / (l * v_up);
-      float* o = a.out + (static_cast<int64_t>(row0 + tok) * a.Hq + head[c]) * D + 4 * fc;
+      float* o = b.out + (static_cast<int64_t>(row0 + 16 * wave + fr) * b.Hq + kv * b.G + g + c) * D + 4 * fc;
 #pragma unroll
       for (int d = 0; d < DT; ++d)
         *reinterpret_cast<f32x4*>(o + 16 * d) = acc[c][d] * inv;
     } else {
-      const int64_t at = part_at(tok, c);
-      float* o = a.part_acc + at * D + 4 * fc;
+      const int64_t at = part_at(16 * wave + fr, c);
+      float* o = b.part_acc + at * D + 4 * fc;
 #pragma unroll
       for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4*>(o + 16 * d) = acc[c][d] * (1.f / v_up);
       if (fc == 0) {
-        a.part_rl[2 * at] = ref[c];  // as the weights used it: any sum with it would round
-        a.part_rl[2 * at + 1] = l;
+        b.part_rl[2 * at] = ref[c];  // as the weights used it: any sum with it would round
+        b.part_rl[2 * at + 1] = l;
       }
     }
   }
   if (redo[0] | redo[1]) {
-    plain_chunk<E, D>(a, kvh, g0, row0, rows, sees, k0, k1, redo, bt,
+    plain_chunk<E, D>(b, work_of(b, unit), kv, g, redo,
                       [&](int t, int c, float m, float l, const float (&v)[D / kWave]) {
                         const int64_t at = part_at(t, c);
-                        float* o = a.out + (static_cast<int64_t>(row0 + t) * a.Hq + kvh * a.G + g0 + c) * D;
+                        float* o = b.out + (static_cast<int64_t>(row0 + t) * b.Hq + kv * b.G + g + c) * D;
 #pragma unroll
                         for (int i = 0; i < D / kWave; ++i) {
                           if (whole)
                             o[lane + kWave * i] = v[i] / l;
                           else
-                            a.part_acc[at * D + lane + kWave * i] = v[i];
+                            b.part_acc[at * D + lane + kWave * i] = v[i];
                         }
                         if (!whole && lane == 0) {
-                          a.part_rl[2 * at] = m;
-                          a.part_rl[2 * at + 1] = l;
+                          b.part_rl[2 * at] = m;
+                          b.part_rl[2 * at + 1] = l;
                         }
                       });
   }
@@ -711,7 +757,7 @@ if constexpr (PL == 1) {
 // Adds the chunks of the tiles that have several: D / 4 lanes per (query token, head).
 //   R = max_j r_j;  out = sum_j 2^(r_j - R) acc_j / sum_j 2^(r_j - R) l_j   (l_j = 0 skipped)
 // Bound by one round trip to memory: four chunks' references, sums and rows are loaded together
-// (one chunk after another the kernel took 34 us for 30 tiles of up to 4 chunks).
+// (one chunk after another the kernel took 34 us for 30 tiles of up to 8 chunks, this way 17).
 template <int D>
 __global__ __launch_bounds__(kWaves* kWave) void prefill_merge_kernel(PrefillArgs a) {
   constexpr int LPR = D / 4, kBatch = 4;
@@ -722,8 +768,6 @@ __global__ __launch_bounds__(kWaves* kWave) void prefill_merge_kernel(PrefillArg
   const int i = blockIdx.x * (kWaves * kWave / LPR) + threadIdx.x / LPR, tok = i / a.Hq, h = i % a.Hq;
   if (n <= 1 || tok >= rows) return;
   const int kvh = h / a.G, g = h % a.G, hp = kvh * a.pairs + g / kHeads, c = g % kHeads;
-  const int64_t base = ((static_cast<int64_t>(tile) * a.Hk * a.pairs + hp) * a.splits * kHeads + c) * kQT + tok;
-  const int64_t step = static_cast<int64_t>(kHeads) * kQT;
   float R = -1e30f, L = 0.f;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
   for (int j0 = 0; j0 < n; j0 += kBatch) {
@@ -731,7 +775,8 @@ __global__ __launch_bounds__(kWaves* kWave) void prefill_merge_kernel(PrefillArg
     f32x4 v[kBatch];
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) {
-      const int64_t at = base + (j0 + j < n ? j0 + j : n - 1) * step;
+      const int64_t at =
+          ((static_cast<int64_t>(part_index(a, tile, min(j0 + j, n - 1))) * a.Hk * a.pairs + hp) * kHeads + c) * kQT + tok;
       r[j] = a.part_rl[2 * at];
       l[j] = a.part_rl[2 * at + 1];
       v[j] = *reinterpret_cast<const f32x4*>(a.part_acc + at * D + 4 * part);
@@ -766,49 +811,93 @@ int device_cus() {
 }
 
 struct ChunkPlan {
-  int chunk, splits;  // chunk tokens (a multiple of 64), most chunks of a tile
+  int chunk, splits, whole;  // as in PrefillArgs
+  int64_t units, parts;      // chunks in all, and of the split tiles
+  int start[kMaxSplits + 1];
 };
 
-// The chunk size by an estimate in context tiles of 64 tokens: a launch of at most two workgroups per
-// CU takes as long as its longest chunk, a larger one its share of the work and half of that; one
-// workgroup per CU runs a tile in 3.2 us, two side by side in 4.8 (2048 tokens, one launch of each);
-// the merge of the chunks costs about 3 tiles. 2048 new tokens, 16 / 8 heads: 115 us in one chunk,
-// 73 at 704 tokens, 83 at 576 (a few workgroups start a second round).
-ChunkPlan plan_chunks(const int64_t* tiles, int64_t n, int64_t groups) {
-  int64_t total = 0, longest = 1;
-  for (int64_t i = 0; i < n; ++i) {
-    const int64_t t = (tiles[4 * i + 1] + tiles[4 * i + 2] - 1 + 63) / 64;
-    total += t;
-    longest = std::max(longest, t);
+// Context tiles (of 64 tokens) of a query tile.
+int context_tiles(const int64_t* t) { return static_cast<int>((t[1] + t[2] - 1 + 63) / 64); }
+
+// Chunks of at most `most` context tiles: where they begin in the launch and in the workspace.
+// `sorted`: the longest contexts first, so that the tiles with more than z chunks are the first ones.
+ChunkPlan lay_out(const int64_t* tiles, int64_t n, int most, int longest, bool sorted) {
+  ChunkPlan p{};
+  p.chunk = most * 64;
+  p.splits = (longest + most - 1) / most;
+  int64_t count[kMaxSplits + 1] = {};  // tiles with exactly so many chunks
+  for (int64_t i = 0; i < n; ++i) ++count[(context_tiles(tiles + 4 * i) + most - 1) / most];
+  int64_t more = n;  // tiles with more than z chunks (not sorted: all, some of them idle)
+  for (int z = 0; z < p.splits; ++z) {
+    if (sorted) more -= count[z];
+    p.start[z] = static_cast<int>(p.units);
+    p.units += more;
+    if (z == 1) p.whole = static_cast<int>(n - more);
   }
-  const int64_t cus = device_cus(), slots = 2 * cus;
-  auto cost = [&](int64_t units, int64_t len, bool merge) {
-    const double one = units <= cus ? 0.67 : 1.0;
-    return (units <= slots ? one * len : static_cast<double>(total * groups) / slots + 0.5 * len) + (merge ? 3.0 : 0.0);
-  };
-  double best = cost(n * groups, longest, false);
-  int64_t take = longest;
-  if (n * groups < 4 * slots) {
-    const int64_t step = std::max<int64_t>(1, longest / 48);
-    for (int64_t c = 4; c < longest; c += step) {
-      int64_t units = 0, len = 1;
-      for (int64_t i = 0; i < n; ++i) {
-        const int64_t t = (tiles[4 * i + 1] + tiles[4 * i + 2] - 1 + 63) / 64, k = (t + c - 1) / c;
-        units += k;
-        len = std::max(len, (t + k - 1) / k);
-      }
-      const double v = cost(units * groups, len, true);
-      if (v < best) {
-        best = v;
-        take = c;
-      }
-    }
-  }
-  return {static_cast<int>(take * 64), static_cast<int>((longest + take - 1) / take)};
+  if (p.splits == 1) p.whole = static_cast<int>(n);
+  for (int z = p.splits; z <= kMaxSplits; ++z) p.start[z] = static_cast<int>(p.units);
+  p.parts = p.units - p.whole;
+  return p;
 }
 
-int64_t partial_floats(int64_t n, int64_t groups, int64_t splits, int64_t D) {
-  return splits > 1 ? n * groups * splits * kHeads * kQT * (D + 2) : 0;
+// The chunk size by an estimate in microseconds: a workgroup takes 7 to start and end, 4.26 per context
+// tile beside another workgroup on its CU and 3.2 alone; up to two per CU the launch takes its longest
+// chunk, above that its work over all places and, where chunks are even, a third of a chunk until the
+// last ones end; the merge takes 6 and the partials' bytes at 8 TB/s. Over 51 batches (64 to 16384 new tokens, up
+// to 100k cached, 8 to 32 heads, both caches; these are the int8 cache's rates at 128 dims, the others scale
+// about alike) the choice is on average 1.7 % and at most 11 % slower than the best of ~20 sizes. 16 / 8 heads,
+// int8, us:
+//   2048 new: 68 in chunks of 704 tokens (256: 87, whole: 118); after 2000 cached 159 in 2048 (896: 145, 256: 213,
+//   whole: 222); after 30000 1081 (8064: 1051, 256: 2011, whole: 1788); 8192 new 566 whole (4096: 589, 256: 1039).
+// Partials take at most kMaxParts bytes, whatever the context.
+constexpr int64_t kMaxParts = 128LL << 20;
+constexpr double kEnds = 7.0, kTile = 4.26, kTileAlone = 3.2, kMerge = 6.0, kBytes = 8e6, kTail = 0.35;
+
+int64_t part_bytes(int64_t parts, int64_t groups, int64_t D) { return parts * groups * kHeads * kQT * (D + 2) * 4; }
+
+ChunkPlan plan_chunks(const int64_t* tiles, int64_t n, int64_t groups, int64_t D) {
+  int64_t total = 0;
+  int longest = 1, before = INT32_MAX;
+  bool sorted = true;
+  for (int64_t i = 0; i < n; ++i) {
+    const int t = context_tiles(tiles + 4 * i);
+    total += t;
+    longest = std::max(longest, t);
+    sorted = sorted && t <= before;
+    before = t;
+  }
+  const double places = 2.0 * device_cus();
+  double best = 0;
+  int take = longest;
+  for (int most = longest; most * kMaxSplits >= longest && most > 0; most -= 1 + most / 12) {
+    const bool split = most < longest;
+    int64_t chunks = n, parts = 0;
+    int len = longest;  // of the longest chunk
+    if (split) {
+      chunks = 0;
+      len = 1;
+      for (int64_t i = 0; i < n; ++i) {
+        const int t = context_tiles(tiles + 4 * i), k = (t + most - 1) / most;
+        chunks += k;
+        parts += k > 1 ? k : 0;
+        len = std::max(len, (t + k - 1) / k);
+      }
+      if (!sorted) chunks = parts = n * ((longest + most - 1) / most);
+      if (chunks >= 65536 || part_bytes(parts, groups, D) > kMaxParts) continue;
+    }
+    const double units = static_cast<double>(chunks * groups), longest_one = kEnds + kTile * len;
+    double us = 2 * units <= places ? kEnds + kTileAlone * len : longest_one;
+    if (units > places)
+      us = std::max(longest_one, (units * kEnds + static_cast<double>(total * groups) * kTile) / places +
+                                     (split ? kTail * longest_one : 0.0));
+    if (split) us += kMerge + static_cast<double>(part_bytes(parts, groups, D)) / kBytes;
+    if (!split || us < best) {
+      best = us;
+      take = most;
+    }
+    if (us > 1.5 * best) break;  // smaller chunks only add to this
+  }
+  return lay_out(tiles, n, take, longest, sorted);
 }
 
 int64_t head_pairs(int64_t Hq, int64_t Hk) { return Hk * ((Hq / Hk + kHeads - 1) / kHeads); }
@@ -819,7 +908,7 @@ extern "C" int64_t llmserve_paged_attention_prefill_workspace_bytes(const int64_
                                                                     int64_t Hq, int64_t Hk, int64_t D) {
   if (n_tiles <= 0 || Hq <= 0 || Hk <= 0 || Hq % Hk || tiles_host == nullptr) return 0;
   const int64_t groups = head_pairs(Hq, Hk);
-  return partial_floats(n_tiles, groups, plan_chunks(tiles_host, n_tiles, groups).splits, D) * 4;
+  return part_bytes(plan_chunks(tiles_host, n_tiles, groups, D).parts, groups, D);
 }
 
 extern "C" int llmserve_paged_attention_prefill(const float* q, const void* k_cache, const void* v_cache,
@@ -852,11 +941,11 @@ extern "C" int llmserve_paged_attention_prefill(const float* q, const void* k_ca
   a.G = static_cast<int>(Hq / Hk);
   a.pairs = (a.G + kHeads - 1) / kHeads;
   const int64_t groups = Hk * a.pairs;
-  const ChunkPlan plan = plan_chunks(tiles_host, n_tiles, groups);
-  const int64_t floats = partial_floats(n_tiles, groups, plan.splits, D);
-  LSH_CHECK(floats == 0 || (workspace != nullptr && workspace_bytes >= floats * 4 && lsh::aligned16(workspace)),
+  const ChunkPlan plan = plan_chunks(tiles_host, n_tiles, groups, D);
+  const int64_t need = part_bytes(plan.parts, groups, D);
+  LSH_CHECK(need == 0 || (workspace != nullptr && workspace_bytes >= need && lsh::aligned16(workspace)),
             "paged_attention_prefill: a 16-byte aligned workspace of %lld bytes is needed (%lld given)",
-            (long long)(floats * 4), (long long)workspace_bytes);
+            (long long)need, (long long)workspace_bytes);
   a.q = q;
   a.kc = k_cache;
   a.vc = v_cache;
@@ -867,9 +956,8 @@ extern "C" int llmserve_paged_attention_prefill(const float* q, const void* k_ca
   a.q_mult = q_mult;
   a.out = out;
   a.part_acc = static_cast<float*>(workspace);
-  a.part_rl = a.part_acc + floats / (D + 2) * D;
+  a.part_rl = a.part_acc + need / 4 / (D + 2) * D;
   a.num_slots = num_slots;
-  a.n_tiles = static_cast<int>(n_tiles);
   a.Hq = static_cast<int>(Hq);
   a.Hk = static_cast<int>(Hk);
   a.max_blocks = static_cast<int>(max_blocks);
@@ -879,9 +967,11 @@ extern "C" int llmserve_paged_attention_prefill(const float* q, const void* k_ca
     if ((1LL << sh) == block_size) a.bs_shift = sh;
   a.chunk = plan.chunk;
   a.splits = plan.splits;
+  a.whole = plan.whole;
+  std::copy(plan.start, plan.start + kMaxSplits + 1, a.start);
   a.scale = scale;
   hipStream_t st = lsh::as_stream(stream);
-  const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(n_tiles), static_cast<unsigned>(plan.splits));
+  const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(plan.units));
   const dim3 block(kWaves * kWave);
   const bool once = plan.splits == 1;
   if (k_scale != nullptr && D == 128)

@@ -110,3 +110,25 @@ def test_single_hip_runtime_with_torch():
     capi()
     maps = {line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line}
     assert len(maps) == 1, maps
+
+
+@pytest.mark.parametrize("heads", [(16, 8, 128), (64, 8, 128), (32, 4, 128), (8, 1, 64), (9, 3, 64)])
+def test_prefill_workspace_is_bounded(lib, heads):
+    """The partials of context chunks stay under 128 MB whatever the prompt and the context, and a long
+    context of few tokens is still split; tiles in any order."""
+    import numpy as np
+
+    def bytes_of(tiles):
+        t = np.ascontiguousarray(tiles, dtype=np.int64)
+        return lib.llmserve_paged_attention_prefill_workspace_bytes(t.ctypes.data, len(t), *heads)
+
+    def tiles_of(new, ctx):
+        t = [(a, min(64, new - a), ctx - new + a + 1, 0) for a in range(0, new, 64)]
+        return sorted(t, key=lambda r: -(r[1] + r[2]))
+
+    for new, cached in [(64, 0), (512, 512), (2048, 0), (2048, 30000), (2048, 120000), (8192, 0), (8128, 120000),
+                        (16384, 0), (40000, 0), (100, 1 << 20)]:
+        tiles = tiles_of(new, new + cached)
+        for order in (tiles, tiles[::-1], tiles[1::2] + tiles[::2]):
+            assert 0 <= bytes_of(order) <= 128 << 20, (new, cached)
+    assert bytes_of(tiles_of(64, 64)) == 0 and bytes_of(tiles_of(64, 30000)) > 0

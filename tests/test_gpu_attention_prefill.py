@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+import capi_util as cu
 from llmserve import attention as at
 from llmserve.kernels import load_paged_attention
 from oracle import math_ref as mr
@@ -185,3 +186,26 @@ def test_infinities_stay_where_they_are(gpu, int8, q_lens, ctx, geom):
     assert np.linalg.norm(got[fine] - want[fine]) <= 2e-6 * np.linalg.norm(want[fine])
     last = want[q_lens[0] - 2: q_lens[0], : geom[0] // geom[1]]
     assert np.isinf(want).any() and (int8 or (np.isfinite(last).any() and np.isnan(last).any()))
+
+
+# many chunks of one tile beside tiles of one chunk, more chunks than a merge round takes, a context of
+# about the most chunks; tiles out of order
+@pytest.mark.parametrize("q_lens,ctx,geom,order", [
+    ([700, 20, 130], [700, 3000, 400], (4, 2, 64, 16), 1), ([700, 20, 130], [700, 3000, 400], (4, 2, 64, 16), -1),
+    ([20], [17000], (2, 1, 128, 16), 1), ([300, 300], [300, 1500], (6, 2, 128, 16), -1)])
+def test_chunks_of_ragged_tiles(gpu, q_lens, ctx, geom, order):
+    q, k, v, tables, meta, dev, mult = make(11, q_lens, ctx, geom, True)
+    tiles = meta.prefill_tiles_host.flip(0) if order < 0 else meta.prefill_tiles_host
+    tiles = tiles.contiguous()
+    lib, d = cu.capi(), geom[2]
+    need = lib.llmserve_paged_attention_prefill_workspace_bytes(tiles.data_ptr(), len(tiles), *geom[:3])
+    assert need > 0  # some tile is split
+    qd, td, md = torch.from_numpy(q).cuda(), tiles.cuda(), torch.from_numpy(mult).cuda()
+    out = torch.full((q.size + 4096,), -7.5, device="cuda")
+    ws = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    cu.check(lib.llmserve_paged_attention_prefill(
+        cu._p(qd), *(cu._p(t) for t in dev), cu._p(meta.block_tables), len(ctx), cu._p(td), tiles.data_ptr(), len(tiles),
+        cu._p(out), len(q), *geom[:3], dev[0].shape[0], meta.block_tables.shape[1], geom[3], d ** -0.5, cu._p(md),
+        cu._p(ws), need, cu._stream()))
+    assert (out[q.size:] == -7.5).all() and (ws[need:] == 0x5A).all()
+    close(out[: q.size].view(q.shape), reference(q, k, v, q_lens, ctx, tables, geom, mult))
