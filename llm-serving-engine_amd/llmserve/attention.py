@@ -471,13 +471,26 @@ def _attend_torch(q: torch.Tensor, k_cache, v_cache, meta: AttentionMetadata, sc
     out[idx] = od.squeeze(1)
 
 
+# Few heads: where an int8 cache's tiles hold at most FEW_ROWS (query token, head pair) rows, the row kernel
+# spreads a context from FEW_CTX tokens on over the device, and a tile's chunks don't (rows / tiles, us):
+# 1 head of 64, 64 tokens in 4096: 14 / 21, in 1024: 11 / 12, in 256: 10 / 8; 128 in 4096: 21 / 21; 2 query heads
+# of 64, 64 in 4096: 17 / 22; 4 / 2 of 128, 32 in 4096: 22 / 24. (fp32 caches: 1 head, 64 in 4096: 30 / 25.)
+FEW_ROWS, FEW_CTX = 64, 512
+
+
 def _tiles_ok(q: torch.Tensor, k: torch.Tensor, meta: AttentionMetadata) -> bool:
     """Whether the tiled prefill kernel takes the batch's tiles; the row kernel has the rest."""
     t, hq, d = q.shape
     hk, bs = k.shape[1], meta.block_size
-    return (d in (64, 128) and hq % hk == 0 and hq // hk <= 8
+    # (up to 8 query heads per kv head: the row kernel, which the other tokens need, has no more)
+    if not (d in (64, 128) and hq % hk == 0 and hq // hk <= 8
             and t < 2**24 and hk <= 4096 and len(meta.prefill_tiles_host) < 65536
-            and meta.block_tables.shape[1] * bs < 2**30 and k.shape[0] * hk < 2**31)
+            and meta.block_tables.shape[1] * bs < 2**30 and k.shape[0] * hk < 2**31):
+        return False
+    tiled = t if meta.rest_rows is None else t - meta.rest_rows.numel()
+    if k.dtype != torch.int8 or tiled * hk * ((hq // hk + 1) // 2) > FEW_ROWS:
+        return True
+    return int(meta.prefill_tiles_host[0, 1:3].sum()) - 1 < FEW_CTX  # (the longest context is first)
 
 
 def _attend_native(ops, q: torch.Tensor, cache, q_mult, meta: AttentionMetadata,

@@ -575,3 +575,19 @@ def test_int4_tile_op_under_transforms():
         assert y.requires_grad and len(calls) == 3
     finally:
         lib._destroy()
+
+
+@pytest.mark.parametrize("heads,new,ctx,int8,tiles", [
+    ((1, 1, 64), 64, 4096, True, False), ((1, 1, 64), 65, 4096, True, True), ((1, 1, 64), 64, 511, True, True),
+    ((1, 1, 64), 64, 512, True, False), ((1, 1, 64), 64, 4096, False, True), ((4, 2, 128), 32, 4096, True, False),
+    ((4, 2, 128), 33, 4096, True, True), ((3, 1, 64), 33, 4096, True, True), ((16, 8, 128), 32, 4096, True, True)])
+def test_few_heads_over_a_long_int8_context_keep_the_row_kernel(heads, new, ctx, int8, tiles):
+    from llmserve import attention as at
+
+    hq, hk, d = heads
+    meta = AttentionMetadata(slot_mapping=torch.empty(0), block_tables=torch.zeros(1, 256, dtype=torch.long),
+                             prefill_tiles_host=torch.tensor([[0, new, ctx - new + 1, 0]]))
+    k = torch.zeros(16, hk, d, dtype=torch.int8 if int8 else torch.float32)
+    assert at._tiles_ok(torch.zeros(new, hq, d), k, meta) == tiles
+    meta.rest_rows = torch.arange(5)  # five of the tokens are in no tile
+    assert at._tiles_ok(torch.zeros(new + 5, hq, d), k, meta) == tiles
