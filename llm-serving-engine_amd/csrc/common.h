@@ -21,6 +21,9 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // Checks the status of the launch just enqueued.
 int launch_status(const char* what);
 
+// CUs of the current device (asked once per device: the linears need it on every call).
+int device_cus();
+
 // Events armed by llmserve_time_next_call() for the calling thread.
 struct TimingEvents {
   hipEvent_t start = nullptr;

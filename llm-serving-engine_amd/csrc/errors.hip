@@ -1,4 +1,5 @@
-// Error reporting of the C ABI: a thread-local message for the last failed call.
+// Error reporting of the C ABI (a thread-local message for the last failed call), and the device's size.
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 
@@ -27,6 +28,18 @@ int launch_status(const char* what) {
     return LLMSERVE_ERR_HIP;
   }
   return LLMSERVE_OK;
+}
+
+int device_cus() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  int cus = cached[dev].load(std::memory_order_relaxed);
+  if (cus == 0) {
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+    cached[dev].store(cus, std::memory_order_relaxed);
+  }
+  return cus;
 }
 
 }  // namespace lsh

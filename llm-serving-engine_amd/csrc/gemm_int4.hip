@@ -762,12 +762,11 @@ void launch_x(const Int4GemmXArgs& a, int64_t slabs, int planes, hipStream_t st)
     lsh::launch(int4_gemm_x<S, NT, false, CO>, grid, block, lds, st, true, a);
 }
 
-int device_cus();
 
 // Tiles per workgroup of the one-tile GEMM: one while the output's 16-column tiles fit the
 // CUs, two beyond (a workgroup converts its x blocks once for both tiles; with one tile per
 // workgroup config 2's gate_up, 384 tiles, puts two workgroups on half the CUs).
-int x_tile_nt(int64_t slabs) { return slabs * kNT > device_cus() ? 2 : 1; }
+int x_tile_nt(int64_t slabs) { return slabs * kNT > lsh::device_cus() ? 2 : 1; }
 
 // S: wavefronts to cover the K blocks in one round (up to 16: K = 2048; K = 3072 takes two
 // rounds); NT: tiles per workgroup (x_tile_nt). More workgroups beat less redundant conversion
@@ -800,21 +799,6 @@ bool launch_x_tile(const Int4GemmXArgs& a, int64_t slabs, int planes, hipStream_
 
 int64_t xsum_rows(int64_t M) { return (M + kRows - 1) / kRows * kRows; }
 
-// CUs of the current device (cached per device: the linears ask on every call).
-int device_cus() {
-  static int cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  if (cached[dev] == 0) {
-    int c = 0;
-    cached[dev] = hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) ==
-                              hipSuccess && c > 0
-                      ? c
-                      : 256;
-  }
-  return cached[dev];
-}
-
 // K planes of the one-launch GEMM (one 16-row tile): a narrow output, whose tiles alone leave
 // most CUs idle and whose every workgroup converts x for all its K blocks, splits the blocks
 // across workgroups: the largest P <= 4 with tiles x P <= CUs, at least 4 blocks in every
@@ -825,7 +809,7 @@ int packed_planes(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || M > kRows || K % kBlk != 0) return 1;
   const int64_t nb = K / kBlk, slabs = pk_slabs(N);
   const int64_t tiles = slabs * (kNT / x_tile_nt(slabs));
-  const int64_t cus = device_cus(), room = lsh::frag_bytes(M, K);
+  const int64_t cus = lsh::device_cus(), room = lsh::frag_bytes(M, K);
   for (int P = 4; P >= 2; --P) {  // plane_sum_kernel adds at most 4
     const int64_t bpp = (nb + P - 1) / P;
     if (tiles * P <= cus && bpp >= 4 && (nb + bpp - 1) / bpp == P &&
@@ -857,7 +841,7 @@ bool launch_lat(const Int4GemmArgs& a, int64_t slabs, int64_t mtiles, int nb_all
   // very wide outputs (at least 256 slabs) with K = 512 or 1024: int4_gemm_wide, about two
   // workgroups per CU
   if (planes == 1 && (nb_all == 4 || nb_all == 8) && slabs >= 256 && slabs * mtiles >= kWideTiles) {
-    const int cus = device_cus();
+    const int cus = lsh::device_cus();
     int64_t groups = (2 * cus + mtiles - 1) / mtiles;
     groups = std::min<int64_t>(groups, slabs / 2);
     groups = std::max<int64_t>(8, (groups + 7) / 8 * 8);
@@ -1121,7 +1105,7 @@ extern "C" int llmserve_int4_linear_gemm_xfrag(const void* xfrag, const void* pa
 extern "C" int64_t llmserve_int4_xfrag_splits(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K < kBlk) return 1;
   const int64_t tiles = pk_slabs(N) * ((M + kRows - 1) / kRows), nb = K / kBlk;
-  const int64_t cus = device_cus();
+  const int64_t cus = lsh::device_cus();
   int64_t P = 1;
   while (P < kMaxPlanes && tiles * 2 * P <= cus && nb >= 4 * 2 * P) P *= 2;
   return P;

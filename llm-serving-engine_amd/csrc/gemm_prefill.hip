@@ -248,28 +248,18 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ p
   }
 }
 
-// K splits for an M x N x K problem: enough (tile, split) units to give every CU one, at most
-// kMaxSplits, each split a multiple of kBK.
-int device_cus() {
-  int cus = 256, dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess) {
-    int c = 0;
-    if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && c > 0)
-      cus = c;
-  }
-  return cus;
-}
-
 // Tile width: 192 when 256-wide tiles leave CUs idle and 192-wide ones fill between 3/4 and
 // all of them (qkv at config 3: 192 -> 256 tiles), else 256.
 int pick_bn(int64_t M, int64_t N) {
-  const int64_t cus = device_cus(), tm = (M + kBM - 1) / kBM;
+  const int64_t cus = lsh::device_cus(), tm = (M + kBM - 1) / kBM;
   const int64_t t256 = tm * ((N + 255) / 256), t192 = tm * ((N + 191) / 192);
   return (t256 < cus && 4 * t192 > 3 * cus && t192 <= cus) ? 192 : 256;
 }
 
+// K splits for an M x N x K problem: enough (tile, split) units to give every CU one, at most
+// kMaxSplits, each split a multiple of kBK.
 int prefill_splits(int64_t M, int64_t N, int64_t K) {
-  const int cus = device_cus();
+  const int cus = lsh::device_cus();
   const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + pick_bn(M, N) - 1) / pick_bn(M, N));
   int s = 1;
   while (s < kMaxSplits && tiles * s * 2 <= cus && K % (static_cast<int64_t>(2 * s) * kBK) == 0) s *= 2;

@@ -690,14 +690,6 @@ void launch_tile(const float* x, const float* inv, const WeightIn& in, TileArgs 
               dim3(kWaves * kWave), 0, st, true, a);
 }
 
-int device_cus() {
-  int dev = 0, c = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0)
-    return 256;
-  return c;
-}
-
 // Tile by the number of workgroups it leaves (256 CUs; us per call, split pass included):
 //   64 x 256, no K split, from 1.25 workgroups per CU: 2048 x 6144 x 1024 63 (32 x 128: 83, 16 x 64:
 //     ~160), 1024 x 6144 x 1024 42 (46);
@@ -709,7 +701,7 @@ void run_tile(const float* x, const float* inv, const WeightIn& in, const TileAr
   auto tiles = [&](int rows, int cols) {
     return static_cast<int64_t>((a.M + rows - 1) / rows) * ((a.N + cols - 1) / cols);
   };
-  const int cus = device_cus();
+  const int cus = lsh::device_cus();
   if (tiles(64, 256) * 4 >= 5 * cus)
     launch_tile<O, 4, 4>(x, inv, in, a, st);
   else if (tiles(32, 128) * 4 >= 3 * cus)

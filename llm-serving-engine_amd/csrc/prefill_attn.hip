@@ -802,14 +802,6 @@ __global__ __launch_bounds__(kWaves* kWave) void prefill_merge_kernel(PrefillArg
       o * inv;
 }
 
-int device_cus() {
-  int dev = 0, c = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0)
-    return 256;
-  return c;
-}
-
 struct ChunkPlan {
   int chunk, splits, whole;  // as in PrefillArgs
   int64_t units, parts;      // chunks in all, and of the split tiles
@@ -866,7 +858,7 @@ ChunkPlan plan_chunks(const int64_t* tiles, int64_t n, int64_t groups, int64_t D
     sorted = sorted && t <= before;
     before = t;
   }
-  const double places = 2.0 * device_cus();
+  const double places = 2.0 * lsh::device_cus();
   double best = 0;
   int take = longest;
   for (int most = longest; most * kMaxSplits >= longest && most > 0; most -= 1 + most / 12) {
