@@ -77,8 +77,6 @@ struct SplitOut {
   float* s;        // ... and its constants
 };
 
-inline int64_t scale_bytes(int64_t M) { return pad_rows(M) * 4; }
-inline int64_t frag_bytes(int64_t M, int64_t K, int P) { return pad_rows(M) * pad_blocks(K, 4) * kBlk * 2 * P; }
 inline int64_t sum_bytes(int64_t rows, int64_t K) { return rows * sum_steps((K + 63) / 64) * 32 * 2 * 2; }
 __host__ __device__ inline int64_t slabs_of(int64_t N) { return (N + 63) / 64; }
 inline int64_t weight_bytes(int64_t N, int64_t K) { return slabs_of(N) * 64 * K / 2; }

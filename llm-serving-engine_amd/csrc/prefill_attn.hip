@@ -678,7 +678,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
         f16x8 vf[PL];
 #pragma unroll
         for (int q = 0; q < PL; ++q) vf[q] = *reinterpret_cast<const f16x8*>(p + q * DT * VS * kFrag);
-if constexpr (PL == 1) {
+        if constexpr (PL == 1) {
 #pragma unroll
           for (int c = 0; c < kHeads; ++c) acc[c][d] = mfma(vf[0], ph[c], acc[c][d]);
 #pragma unroll
