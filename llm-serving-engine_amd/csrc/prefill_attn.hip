@@ -5,13 +5,13 @@
 // The row kernel (paged_decode.hip) gives every token a query row of its own: it reads the whole
 // context once per token and runs on the VALU (2 prompts of ~900 tokens after ~1000 cached ones and 24
 // decode rows: 962 us). Here a workgroup takes 64 query tokens and two query heads of one kv head and
-// walks the context in tiles of 64 tokens (fp32 cache: 32) that its four wavefronts share: 87 us for
-// the two prompts, 1000 new tokens over the fp32 cache 776 -> 64.
+// walks the context in tiles of 64 tokens (fp32 cache: 32) that its four wavefronts share: 75 us for
+// the two prompts, 1000 new tokens over the fp32 cache 776 -> 51.
 //
 // Precision is fp32's: q, the weights and fp32 K / V rows are each split into two fp16 pieces (22
 // bits) after scaling by a power of two (per query row and head, per cache row); int8 codes are exact
 // in fp16, their scales stay in fp32 on the score and on the weight. Products are exact and summed in
-// fp32. Measured against float64, 1000 new tokens: int8 1.5e-7, fp32 1.6e-7 (the row kernel 3.0e-7, 1.6e-7).
+// fp32. Measured against float64, 1000 new tokens: int8 1.2e-7, fp32 1.6e-7 (the row kernel 1.7e-7, 1.6e-7).
 //
 // Both products are transposed: S^T = K Q^T leaves lane (fr, fc) the scores of query fr for tokens
 // 16 tt + 4 fc + e, which is the B operand layout of O^T = V^T P^T when the k order of that product is
@@ -23,9 +23,9 @@
 // current one is computed, then widens it into MFMA fragments (positions in a fragment are permuted so
 // that neither the writes nor the reads conflict). Long contexts are split into chunks where the
 // tiles alone would leave CUs idle, and a second launch adds the chunks.
-// What bounds it: per context tile a wavefront issues 128 products (2048 matrix-core cycles) and ~410
-// VALU instructions (exp, the splits, widening); the two wavefronts of a SIMD overlap them only in
-// part: 8192 tokens run at 460 TFLOP/s of attention, 0.92 PFLOP/s of fp16 products.
+// What bounds it: per context tile a wavefront issues 128 products (2048 matrix-core cycles) and about 500
+// VALU instructions (exp, the splits, widening, the sums); the two wavefronts of a SIMD overlap them
+// only in part: 8192 tokens, in one chunk, run at 500 TFLOP/s of attention, 1 PFLOP/s of fp16 products.
 #include <algorithm>
 #include <type_traits>
 
@@ -639,9 +639,9 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
       }
     }
     // weights and their product with V
+    f16x8 ph[VS][kHeads], pl[VS][kHeads];
 #pragma unroll
     for (int vs = 0; vs < VS; ++vs) {
-      f16x8 ph[kHeads], pl[kHeads];
       f32x4 vsc[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -668,33 +668,41 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void prefill_kernel(PrefillArgs a
           lo[2 * h + 1] = l1;
         }
         sum[c] += eight;
-        ph[c] = __builtin_bit_cast(f16x8, hi);
-        pl[c] = __builtin_bit_cast(f16x8, lo);
+        ph[vs][c] = __builtin_bit_cast(f16x8, hi);
+        pl[vs][c] = __builtin_bit_cast(f16x8, lo);
       }
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int d = 0; d < DT; ++d) {
-        const char* p = base + kKBytes + (d * VS + vs) * kFrag + ((fr ^ (d % 8)) + 16 * fc) * 16;
-        f16x8 vf[PL];
-#pragma unroll
-        for (int q = 0; q < PL; ++q) vf[q] = *reinterpret_cast<const f16x8*>(p + q * DT * VS * kFrag);
-        if constexpr (PL == 1) {
-#pragma unroll
-          for (int c = 0; c < kHeads; ++c) acc[c][d] = mfma(vf[0], ph[c], acc[c][d]);
-#pragma unroll
-          for (int c = 0; c < kHeads; ++c) acc[c][d] = mfma(vf[0], pl[c], acc[c][d]);
-        } else {  // the tile's sum apart, its small products first: one rounding at acc's size
-          f32x4 t[kHeads];
-#pragma unroll
-          for (int c = 0; c < kHeads; ++c) t[c] = mfma(vf[PL - 1], ph[c], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-          for (int c = 0; c < kHeads; ++c) t[c] = mfma(vf[0], pl[c], t[c]);
-#pragma unroll
-          for (int c = 0; c < kHeads; ++c) acc[c][d] += mfma(vf[0], ph[c], t[c]);
-        }
-      }
-      __builtin_amdgcn_s_setprio(0);
     }
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      f16x8 vf[VS][PL];
+#pragma unroll
+      for (int vs = 0; vs < VS; ++vs)
+#pragma unroll
+        for (int q = 0; q < PL; ++q)
+          vf[vs][q] = *reinterpret_cast<const f16x8*>(base + kKBytes + (d * VS + vs) * kFrag +
+                                                      ((fr ^ (d % 8)) + 16 * fc) * 16 + q * DT * VS * kFrag);
+      // The tile's sum apart, its small products first: one rounding at acc's size (summed into acc product
+      // by product, int8, the error against float64 was 1.2e-6 for 2048 tokens after 30000, now 3.6e-7;
+      // for 2048 2.0e-7, now 1.4e-7; row kernel 5.3e-7 and 1.9e-7; at the same speed).
+      f32x4 t[kHeads] = {};
+#pragma unroll
+      for (int vs = 0; vs < VS; ++vs) {
+        if constexpr (PL == 2) {
+#pragma unroll
+          for (int c = 0; c < kHeads; ++c) t[c] = mfma(vf[vs][PL - 1], ph[vs][c], t[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < kHeads; ++c) t[c] = mfma(vf[vs][0], pl[vs][c], t[c]);
+      }
+#pragma unroll
+      for (int vs = 0; vs < VS; ++vs)
+#pragma unroll
+        for (int c = 0; c < kHeads; ++c) t[c] = mfma(vf[vs][0], ph[vs][c], t[c]);
+#pragma unroll
+      for (int c = 0; c < kHeads; ++c) acc[c][d] += t[c];
+    }
+    __builtin_amdgcn_s_setprio(0);
   }
 
   // ---- output: lane (fr, fc) holds dims 16 d + 4 fc + e of its query -----------------------------
