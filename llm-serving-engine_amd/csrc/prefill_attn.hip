@@ -5,7 +5,7 @@
 // The row kernel (paged_decode.hip) gives every token a query row of its own: it reads the whole
 // context once per token and runs on the VALU (2 prompts of ~900 tokens after ~1000 cached ones and 24
 // decode rows: 962 us). Here a workgroup takes 64 query tokens and two query heads of one kv head and
-// walks the context in tiles of 64 tokens (fp32 cache: 32) that its four wavefronts share: 75 us for
+// walks the context in tiles of 64 tokens (fp32 cache: 32) that its four wavefronts share: 79 us for
 // the two prompts, 1000 new tokens over the fp32 cache 776 -> 51.
 //
 // Precision is fp32's: q, the weights and fp32 K / V rows are each split into two fp16 pieces (22
