@@ -303,7 +303,8 @@ __device__ __forceinline__ void segment_state(const DecodeArgs& a, int b, int h,
     };
 
     // One step. A row outside the segment or the cache gets the score -inf (p = 0, and it
-    // never raises the max) and the value scale 0 (its bytes, whatever they hold, add 0).
+    // never raises the max) and the value scale 0 (its int8 codes add 0; fp32 values, which may be
+    // infinite or NaN in a slot that no token of the row fills, are cleared).
     auto consume = [&](const Tok<E>& c) {
       float kf[16];
       unpack16(c.k, kf);
@@ -332,6 +333,12 @@ __device__ __forceinline__ void segment_state(const DecodeArgs& a, int b, int h,
       }
       float vf[16];
       unpack16(c.v, vf);
+      if constexpr (kF32) {
+        if (__builtin_amdgcn_ballot_w64(!c.valid)) {  // a segment's ends, blocks outside the cache
+#pragma unroll
+          for (int i = 0; i < 16; ++i) vf[i] = c.valid ? vf[i] : 0.f;
+        }
+      }
       const float vsc = c.valid ? c.vs : 0.f;
 #pragma unroll
       for (int g = 0; g < G; ++g) {

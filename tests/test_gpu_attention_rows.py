@@ -217,3 +217,25 @@ def test_loader_v1_entry_and_simd_switch(gpu, simd, partition):
     torch.testing.assert_close(out, ref, atol=1e-5, rtol=1e-5)
     ref64 = mr.paged_decode_f64(*arrays, bs, sc)
     cu.assert_rel_close(ref, ref64, TOL, "v1 vs f64")
+
+
+@pytest.mark.parametrize("geom", [(16, 8, 128, 16), (4, 4, 64, 16), (6, 2, 64, 5), (8, 1, 128, 1), (2, 1, 32, 64)])
+def test_slots_that_no_row_sees_may_hold_anything(gpu, geom):
+    """An fp32 cache's slots past a context, and blocks of no sequence, may hold infinities and NaN (what
+    an earlier owner left): the rows' results are the same bits as over zeros there."""
+    hq, hk, d, bs = geom
+    ctx = [1, 7, 300, 33, 1000, 64]
+    rng, tables, total = _batch(sum(geom), [1] * len(ctx), ctx, bs)
+    bt = _packed(tables, ctx, bs)
+    seen = np.zeros(total * bs, bool)
+    for row, c in zip(bt, ctx):
+        t = np.arange(c)
+        seen[row[t // bs] * bs + t % bs] = True
+    k, v = (cu.dev(rng.standard_normal((total * bs, hk, d)).astype(F32)) for _ in range(2))
+    q, unseen = cu.dev(rng.standard_normal((len(ctx), hq, d)).astype(F32)), cu.dev(~seen)
+    outs = []
+    for fill in (0.0, float("nan"), float("inf")):
+        k[unseen], v[unseen] = fill, fill
+        outs.append(cu.paged_decode_f32(q, k, v, cu.dev(bt), cu.dev(np.array(ctx)), bs, d ** -0.5))
+    assert unseen.any() and outs[0].isfinite().all()
+    assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
