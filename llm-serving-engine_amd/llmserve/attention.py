@@ -36,9 +36,10 @@ QUERY_TILE = 64  # query tokens of a prefill tile
 # Which tokens go to the prefill kernel: those of sequences with at least TILE_ROWS new ones, where
 # the row kernel's work on them, sum(new * context), at ROW_US per token outweighs what a tiled launch
 # adds: TILE_US, CTX_US per token of the longest context, and REST_US for a row launch of its own
-# when other tokens remain. Measured at 16 / 8 heads, int8 (rows / tiles, us): one sequence of 32 new
-# tokens in 1024: 21 / 24, 64: 29 / 27, 32 in 4096: 43 / 39, 64 in 256: 17 / 20; eight sequences of 4 in
-# 4096: 47 / 62, of 8: 79 / 61, of 16 in 1024: 50 / 31 (fp32 caches gain from fewer tokens on).
+# when other tokens remain. Measured at 16 / 8 heads, int8 (rows / tiles, us): one sequence of 8 new
+# tokens in 4096: 22 / 26, 16 in 1024: 17 / 15, 32: 21 / 16, 64: 29 / 19, 32 in 4096: 44 / 32, 64 in 256: 17 / 14;
+# four sequences of 8 in 4096: 44 / 33, of 8 in 1024: 21 / 18. The line was drawn when a tile of few tokens
+# took 3 to 8 us more than it does now; it leaves the row kernel batches where that is a few us slower.
 TILE_ROWS = 8
 ROW_US, TILE_US, CTX_US, REST_US = 0.235e-3, 4.0, 6e-3, 20.0
 
