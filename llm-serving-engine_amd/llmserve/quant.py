@@ -344,7 +344,7 @@ class Int4Linear(nn.Module):
             xs = x2 * self.inv_act_scale if self.inv_act_scale is not None else x2
             y = xs @ self.dequantize().t()
         elif path == "gemm":
-            packed = self.gemm_packed
+            packed = self._buffers["gemm_packed"]  # (an attribute lookup costs as much as the check)
             if self.kernel == "gemm" and not self._packed_current():  # "auto" comes here with a current one
                 packed = native.int4_gemm_pack(self.nibbles, self.g_scale, self.g_zero, self.group_size)
             y = native.int4_linear_gemm_packed(x2.contiguous(), packed, self.out_features,
